@@ -98,7 +98,7 @@ __device__ __forceinline__ T PressurePrimM(T E, T d, T vx, T vy, T vz, T g, T bx
 template <typename T>
 __device__ __forceinline__ T EnergyPrimM(T P, T d, T vx, T vy, T vz, T g, T bx, T by, T bz)
 {
-  T e = (Fmax(P, T(kTinyNumber)) / (g - T(1.))) + T(0.5) * d * Dot(vx, vy, vz, vx, vy, vz);
+  T e = QuotOnce(Fmax(P, T(kTinyNumber)), g - T(1.)) + T(0.5) * d * Dot(vx, vy, vz, vx, vy, vz);
   e += MagEnergy(bx, by, bz);
   return e;
 }
@@ -150,9 +150,10 @@ __device__ __forceinline__ PrimM<typename P::T> LoadDataM(const double *U, int x
   const double d = U[id];
   double vx, vy, vz;
   if constexpr (P::kExact) {
-    vx = mx / d, vy = my / d, vz = mz / d;
+    const double r = RcpRefined(d);
+    vx = Quot(mx, d, r), vy = Quot(my, d, r), vz = Quot(mz, d, r);
   } else {
-    const double inv = 1.0 / d;
+    const double inv = QuotOnce(1.0, d);
     vx = mx * inv, vy = my * inv, vz = mz * inv;
   }
   const double p = PressurePrimM(U[4 * n + id], d, vx, vy, vz, g, bx, by, bz);
@@ -182,8 +183,9 @@ __device__ __forceinline__ EigenM<typename P::T> ComputeEigenM(const PrimM<typen
     if (num1 <= T(0.0)) {
       e.af = T(0.0), e.as = T(1.0);
     } else {
-      e.af = Sqrt<P>(Div1<P>(num1, denom));
-      e.as = Sqrt<P>(Div1<P>(num2, denom));
+      const T inv_denom = Rcp<P>(denom);
+      e.af = Sqrt<P>(Div<P>(num1, denom, inv_denom));
+      e.as = Sqrt<P>(Div<P>(num2, denom, inv_denom));
     }
   }
   const T bden = Div1<P>(T(1.0), Sqrt<P>(w.by * w.by + w.bz * w.bz));  // rhypot
@@ -199,8 +201,9 @@ __device__ __forceinline__ EigenM<typename P::T> ComputeEigenM(const PrimM<typen
   e.sqrt_d       = Sqrt<P>(w.d);
   e.Af           = e.af * cs * e.sqrt_d;
   e.As           = e.as * cs * e.sqrt_d;
-  e.Apf          = Div1<P>(T(0.5) * e.af, cs * e.sqrt_d);
-  e.Aps          = Div1<P>(T(0.5) * e.as, cs * e.sqrt_d);
+  const T csd = cs * e.sqrt_d, inv_csd = Rcp<P>(csd);
+  e.Apf          = Div<P>(T(0.5) * e.af, csd, inv_csd);
+  e.Aps          = Div<P>(T(0.5) * e.as, csd, inv_csd);
   return e;
 }
 
@@ -262,7 +265,7 @@ __device__ __forceinline__ T MonoM(T l, T r, T c, T v)  // Monotonize_Characteri
 template <typename T>
 __device__ __forceinline__ T VlM(T l, T r)  // Van_Leer_Slope
 {
-  return (l * r > T(0.0)) ? T(2.0) * l * r / (l + r) : T(0.0);
+  return (l * r > T(0.0)) ? QuotOnce(T(2.0) * l * r, l + r) : T(0.0);
 }
 template <typename T>
 __device__ __forceinline__ void LimitM(T &l, T &r, T vm, T v0, T vp)  // Plm_Limit_Interfaces
@@ -283,10 +286,10 @@ __device__ __forceinline__ void PlmcPrimsM(const PrimM<typename P::T> &cm, const
 {
   using T           = typename P::T;
   const T gg        = T(g);
-  const T inv_d     = Div1<P>(T(1.0), c0.d);
+  const T inv_d     = Rcp<P>(c0.d);
   const T cs        = Sqrt<P>(Div<P>(gg * c0.p, c0.d, inv_d));  // Calc_Sound_Speed
   const T cs2       = cs * cs;
-  const T inv_cs2   = Div1<P>(T(1.0), cs2);
+  const T inv_cs2   = Rcp<P>(cs2);
   const EigenM<T> e = ComputeEigenM<P>(c0, cs, cs2, gg);
   auto slope = [](const PrimM<T> &l, const PrimM<T> &r, T c) {
     return PrimM<T>{c * (r.d - l.d), c * (r.vx - l.vx), c * (r.vy - l.vy), c * (r.vz - l.vz),
@@ -358,10 +361,10 @@ __device__ __forceinline__ void PpmcPrimsM(const PrimM<typename P::T> &cm2, cons
 {
   using T           = typename P::T;
   const T gg        = T(g);
-  const T inv_d     = Div1<P>(T(1.0), c0.d);
+  const T inv_d     = Rcp<P>(c0.d);
   const T cs        = Sqrt<P>(Div<P>(gg * c0.p, c0.d, inv_d));  // Calc_Sound_Speed
   const T cs2       = cs * cs;
-  const T inv_cs2   = Div1<P>(T(1.0), cs2);
+  const T inv_cs2   = Rcp<P>(cs2);
   const EigenM<T> e = ComputeEigenM<P>(c0, cs, cs2, gg);
   const Char7<T> a0  = PrimToCharM<P>(c0, c0, e, cs2, inv_d, inv_cs2);
   const Char7<T> am1 = PrimToCharM<P>(c0, cm1, e, cs2, inv_d, inv_cs2);
@@ -436,7 +439,7 @@ __device__ __forceinline__ HStateM<typename P::T> LoadStateM(const ConsM<typenam
   using T = typename P::T;
   HStateM<T> s;
   s.d       = Fmax(q.d, T(kTinyNumber));
-  const T inv = Div1<P>(T(1.0), s.d);
+  const T inv = Rcp<P>(s.d);
   s.vx      = Div<P>(q.mx, s.d, inv);
   s.vy      = Div<P>(q.my, s.d, inv);
   s.vz      = Div<P>(q.mz, s.d, inv);
@@ -468,12 +471,13 @@ __device__ __forceinline__ HStarM<typename P::T> StarStateM(const HStateM<typena
 {
   using T = typename P::T;
   HStarM<T> o;
-  o.d = Div1<P>(s.d * (side - s.vx), (side - M));
+  const T inv_sm = Rcp<P>(side - M);
+  o.d = Div<P>(s.d * (side - s.vx), (side - M), inv_sm);
   if (Fabs(s.d * (side - s.vx) * (side - M) - (bx * bx)) < ptStar * T(kHlldSmall)) {
     o.vy = s.vy, o.vz = s.vz, o.by = s.by, o.bz = s.bz;
   } else {
     const T denom = s.d * (side - s.vx) * (side - M) - (bx * bx);
-    const T inv   = Div1<P>(T(1.0), denom);
+    const T inv   = Rcp<P>(denom);
     T coef        = Div<P>(bx * (M - s.vx), denom, inv);
     o.vy          = s.vy - s.by * coef;
     o.vz          = s.vz - s.bz * coef;
@@ -483,9 +487,9 @@ __device__ __forceinline__ HStarM<typename P::T> StarStateM(const HStateM<typena
     o.by          = s.by * coef;
     o.bz          = s.bz * coef;
   }
-  o.E = Div1<P>((s.E * (side - s.vx) - s.pt * s.vx + ptStar * M +
-                 bx * (Dot(s.vx, s.vy, s.vz, bx, s.by, s.bz) - Dot(M, o.vy, o.vz, bx, o.by, o.bz))),
-                (side - M));
+  o.E = Div<P>((s.E * (side - s.vx) - s.pt * s.vx + ptStar * M +
+                bx * (Dot(s.vx, s.vy, s.vz, bx, s.by, s.bz) - Dot(M, o.vy, o.vz, bx, o.by, o.bz))),
+               (side - M), inv_sm);
   return o;
 }
 
@@ -740,6 +744,7 @@ __device__ __forceinline__ void CtStageCell(CtPlane<TF, SX, SY> &P, int cx, int 
     P.f[d][2][cy][cx] = Fl[d][size_t(kBx + 1) * n + cid];
   }
   const double d     = U[cid];
+  const double rd    = RcpRefined(d);
   const double m[3]  = {U[n + cid], U[2 * n + cid], U[3 * n + cid]};
   const double b[3]  = {U[5 * n + cid], U[6 * n + cid], U[7 * n + cid]};
   const double bm[3] = {U[5 * n + cid - 1], U[6 * n + cid - sy], U[7 * n + cid - sz]};
@@ -748,7 +753,7 @@ __device__ __forceinline__ void CtStageCell(CtPlane<TF, SX, SY> &P, int cx, int 
     const int m1 = (q + 1) % 3, m2 = (q + 2) % 3;
     const double b2 = 0.5 * (b[m1] + bm[m1]);
     const double b3 = 0.5 * (b[m2] + bm[m2]);
-    P.ec[q][cy][cx] = (m[m2] * b2 - m[m1] * b3) / d;
+    P.ec[q][cy][cx] = Quot(m[m2] * b2 - m[m1] * b3, d, rd);
   }
   if (own) {
     own[0] = d, own[1] = m[0], own[2] = m[1], own[3] = m[2], own[4] = U[4 * n + cid];
@@ -903,10 +908,12 @@ __device__ __forceinline__ double MhdInverseCrossingTimeOf(double d, double mx, 
                                                            double bx, double by, double bz, double dx, double dy,
                                                            double dz, double g)
 {
-  const double dinv = 1.0 / d;
+  const double dinv = QuotOnce(1.0, d);
   const double vx = mx * dinv, vy = my * dinv, vz = mz * dinv;
   const double gasP = PressurePrimM(E, d, vx, vy, vz, g, bx, by, bz);
   const double cf   = Magnetosonic<PolicyExact>(d, gasP, bx, by, bz, g, 1.0);
+  // (compiled divisions: hoisted reciprocals of dx, dy, dz put MhdFlux1MarchKernel into spills,
+  // 0.96 -> 1.03 ms on Orszag-Tang 256^3)
   double m          = Fmax((Fabs(vx) + cf) / dx, (Fabs(vy) + cf) / dy);
   m                 = Fmax(m, (Fabs(vz) + cf) / dz);
   return Fmax(m, 0.0);
@@ -1333,10 +1340,10 @@ __device__ __forceinline__ void FullCell(const MhdArgs &a, double dt, int x, int
     if (mark) {
       MarkRepair(a.rep, id, mark);
     } else if (a.flags & kFlagTemperatureFloor) {
-      const double dinv = 1.0 / un[0];
+      const double rd = RcpRefined(un[0]), dinv = Quot(1.0, un[0], rd);
       const double vx = un[1] * dinv, vy = un[2] * dinv, vz = un[3] * dinv;
       const double Ekin = 0.5 * un[0] * (vx * vx + vy * vy + vz * vz);
-      if ((un[4] - Ekin) / un[0] < a.U_floor) un[4] = Ekin + un[0] * a.U_floor;
+      if (Quot(un[4] - Ekin, un[0], rd) < a.U_floor) un[4] = Ekin + un[0] * a.U_floor;
     }
 #pragma unroll
     for (int f = 0; f < 5; f++) U[size_t(f) * n + id] = un[f];

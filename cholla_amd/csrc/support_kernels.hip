@@ -597,7 +597,7 @@ __global__ void Vl1dStage2Kernel(double *U, const double *W, int n, int ng, doub
   double m        = 0.0;
   const double dt = dt_dev ? *dt_dev : dt_host;
   if (id >= ng && id < n - ng) {
-    const T g = T(gamma), inv_gm1 = T(1.0 / (gamma - 1.0));
+    const T g = T(gamma), inv_gm1 = P::kExact ? T(RcpRefined(gamma - 1.0)) : T(1.0 / (gamma - 1.0));
     double gm = 0.0, gp = 0.0;
     Cons<double> fm, fp;
     if constexpr (RK == kPCM && DE) {
@@ -992,7 +992,7 @@ __global__ void ReconGridKernel(const double *U, double *QL, double *QR, int nx,
     ReconPlmc<PolicyExact>(s, gamma, L, R);
     if constexpr (DE) ReconPlmcScalar<PolicyExact>(ge, gL, gR);
   }
-  const double inv_gm1 = 1.0 / (gamma - 1.0);
+  const double inv_gm1 = Rcp<PolicyExact>(gamma - 1.0);
   auto write = [&](const Prim<double> &q, double *Q, size_t id) {  // Write_Data, reconstruction.h:918-958
     Q[id]           = q.d;
     Q[o1 * nc + id] = q.d * q.vx;

@@ -238,11 +238,12 @@ __device__ __forceinline__ PcmCell<typename P::T, DE> MakePcmCell(double d, doub
   PcmCell<T, DE> c;
   if constexpr (P::kExact) {
     c.d = d, c.mx = mx, c.my = my, c.mz = mz, c.E = E;
-    c.vx = mx / d, c.vy = my / d, c.vz = mz / d;
+    const double r = RcpRefined(d);
+    c.vx = Quot(mx, d, r), c.vy = Quot(my, d, r), c.vz = Quot(mz, d, r);
     c.p = 0;
   } else {
     // FP64 primitive recovery, then narrowing (a no-op for PolicyFast)
-    double inv = 1.0 / d;
+    double inv = Quot(1.0, d, RcpRefined(d));
     double vx = mx * inv, vy = my * inv, vz = mz * inv;
     double p;
     if constexpr (DE) {
@@ -506,13 +507,15 @@ __device__ __forceinline__ void Stage1Tile(const StepArgs &a, int R1, int bx, in
           // PCM hands the conserved half state itself to the Riemann solver (pcm_cuda.cu)
           const bool cons_w = (a.flags & kFlagConservedW) != 0;
           W[id]          = T(uh[0]);
-          W[nc + id]     = cons_w ? T(uh[1]) : T(uh[1] / uh[0]);
-          W[2 * nc + id] = cons_w ? T(uh[2]) : T(uh[2] / uh[0]);
-          W[3 * nc + id] = cons_w ? T(uh[3]) : T(uh[3] / uh[0]);
+          const double rd = RcpRefined(uh[0]);
+          W[nc + id]     = cons_w ? T(uh[1]) : T(Quot(uh[1], uh[0], rd));
+          W[2 * nc + id] = cons_w ? T(uh[2]) : T(Quot(uh[2], uh[0], rd));
+          W[3 * nc + id] = cons_w ? T(uh[3]) : T(Quot(uh[3], uh[0], rd));
           W[4 * nc + id] = T(uh[4]);
           W[5 * nc + id] = T(uh[5]);
         } else {
-          double vx = uh[1] / uh[0], vy = uh[2] / uh[0], vz = uh[3] / uh[0];
+          const double rd = RcpRefined(uh[0]);
+          double vx = Quot(uh[1], uh[0], rd), vy = Quot(uh[2], uh[0], rd), vz = Quot(uh[3], uh[0], rd);
           double E_kin   = 0.5 * uh[0] * SquareMag(vx, vy, vz);
           W[id]          = T(uh[0]);
           W[nc + id]     = T(vx);
@@ -526,7 +529,7 @@ __device__ __forceinline__ void Stage1Tile(const StepArgs &a, int R1, int bx, in
           } else {
             store_p(PressureFromDE(uh[4], uh[4] - E_kin, uh[5], a.gamma));
           }
-          W[kWGasEnergy<P> * nc + id] = T(uh[5] / uh[0]);
+          W[kWGasEnergy<P> * nc + id] = T(Quot(uh[5], uh[0], rd));
         }
       } else {
         Prim<double> w = LoadPrim(uh[0], uh[1], uh[2], uh[3], uh[4], a.gamma);
@@ -970,7 +973,7 @@ __device__ __forceinline__ void Stage2Tile(const StepArgs &a, int bx, int by, in
   const double dtodx = dt / a.dx, dtody = dt / a.dy, dtodz = dt / a.dz;
   const T *W         = reinterpret_cast<const T *>(a.W);
   double *U          = a.U;
-  const double inv_dx = 1.0 / a.dx, inv_dy = 1.0 / a.dy, inv_dz = 1.0 / a.dz;
+  const double inv_dx = CellRcp<P>(a.dx), inv_dy = CellRcp<P>(a.dy), inv_dz = CellRcp<P>(a.dz);
   if (dt == 0.0) return;  // a device-timed step past the output time (uniform per box)
   const bool pf = (a.flags & kFlagPositivityFallback) != 0;
 
@@ -1222,11 +1225,12 @@ __device__ __forceinline__ void Stage2Tile(const StepArgs &a, int bx, int by, in
 #pragma unroll
         for (int q = 0; q < NC; q++) U[q * nc + id] = un[q];
       } else {
-        double dinv = 1.0 / un[0];
+        const double rd = RcpRefined(un[0]);
+        double dinv = Quot(1.0, un[0], rd);
         double vx = un[1] * dinv, vy = un[2] * dinv, vz = un[3] * dinv;
         if (a.flags & kFlagTemperatureFloor) {  // Temperature_Floor_Kernel, hydro_cuda.cu:1132-1146
           double Ekin = 0.5 * un[0] * (vx * vx + vy * vy + vz * vz);
-          double uint = P::kExact ? (un[4] - Ekin) / un[0] : (un[4] - Ekin) * dinv;
+          double uint = P::kExact ? Quot(un[4] - Ekin, un[0], rd) : (un[4] - Ekin) * dinv;
           if (uint < a.U_floor) un[4] = Ekin + un[0] * a.U_floor;
         }
 #pragma unroll
@@ -1462,8 +1466,8 @@ __device__ void RepairBox(const StepArgs &a)
                 a.U[4 * nc + id] = un[4];
               }
               if (a.flags & kFlagReduceDt) {
-                double m_ = InverseCrossingTimeP<P>(un[4], un[0], dinv, vx, vy, vz, a.dx, a.dy, a.dz, 1.0 / a.dx,
-                                                    1.0 / a.dy, 1.0 / a.dz, a.gamma);
+                double m_ = InverseCrossingTimeP<P>(un[4], un[0], dinv, vx, vy, vz, a.dx, a.dy, a.dz,
+                                                    CellRcp<P>(a.dx), CellRcp<P>(a.dy), CellRcp<P>(a.dz), a.gamma);
                 atomicMax(a.dti, (unsigned long long)__double_as_longlong(m_));
               }
               if (a.flags & kFlagPeriodicGhosts) WritePeriodicImages<5>(a.U, nc, nx, ny, nz, ng, i, j, k, un);
