@@ -91,8 +91,6 @@ int SolverKind(int riemann)
   return chl::kRiemannHllc;
 }
 
-int DefaultChunk(int n_real) { return std::max(8, std::min(n_real, 32)); }
-
 // Gravity records a step keeps for repaired cells (static gravity only).
 constexpr int kRepairGravCap = 4096;
 
@@ -343,15 +341,69 @@ size_t chl_capi::HalfStepBytes(const chl_hydro_config &c, size_t *w_main)
   return main_ + (c.dual_energy ? n * sizeof(double) : 0);
 }
 
+// A workgroup marches kchunk planes, so a box of few tiles needs short chunks to fill the 256
+// CUs, while a large one wants long chunks: each chunk starts with work its neighbour repeats
+// (c0 planes' worth) and re-reads its halo planes.  The shape taken has the least
+// rounds x (kchunk + c0), rounds being the workgroups over the slots they run in: whole rounds
+// for the first few, and half a round of tail after that.  Measured against the best of every
+// tile and z-chunk on boxes of 32^3 to 384^3 the pick is 1-5 % off in the mean and 29 % at
+// worst; the 32-plane chunks of one fixed tile it replaced left a 48^3 box to 12-18 workgroups
+// (stage 1 / 2, PLMC, reference order: 209 / 406 us against 22 / 34) and KH 512^3 (mixed) on
+// stage-2 tiles of 16x8 (10.2 ms against 8.5).
+//   tiles    stage 1: 16x16 (FP64), 32x8 (mixed: KH 256^3 495 against 536 us); stage 2: 16x16,
+//            and 32x16 in the FP64 forms where it rounds better (with PLMC it needs 5 % less:
+//            KH 256^3 1.89 against 2.09 ms), or 16x8 where those leave CUs idle (32^3, PPMC,
+//            fast form: 27 against 28 us), which the narrow kernels do not have
+//   caps     stage 1 loses to its z planes leaving the L2 past 8 (FP64) or 16 planes; stage 2
+//            past 32, with dual energy past 8
+void chl_capi::PickLaunchShape(int stage, int precision, int reconstruction, bool dual_energy, bool narrow,
+                               const std::vector<StageExtent> &boxes, int &tile, int &kchunk)
+{
+  const bool mixed = precision == CHL_PREC_MIXED;
+  const int cus    = 256;  // gfx950
+  const int waves  = stage == 1 ? 4 : (mixed ? 3 : 2);  // per SIMD
+  const int cap    = stage == 1 ? (mixed ? 16 : 8) : (dual_energy ? 8 : 32);
+  const double c0  = stage == 1 ? 1.0 : 0.5;
+  const bool all   = stage == 2 && !mixed && !narrow;
+  int tiles[3]     = {stage == 1 && mixed ? 0 : 1, all ? 3 : -1, all ? 4 : -1};
+  if (all) std::swap(tiles[0], tiles[1]);  // equal costs: the first
+  if (tile >= 0) tiles[0] = tile, tiles[1] = tiles[2] = -1;
+  static const int kChunks[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
+  double best = std::numeric_limits<double>::infinity();
+  int best_t = tiles[0], best_k = kchunk > 0 ? kchunk : 1;
+  for (int t : tiles) {
+    if (t < 0 || t >= chl::kNumTiles) continue;
+    const chl::TileShape s = chl::kTiles[t];
+    const double slots     = t == 3 && tile < 0 ? cus : double(cus) * std::max(1, 4 * waves * 64 / (s.tx * s.ty));
+    const double weight    = t == 4 && reconstruction == CHL_RECON_PLMC ? 0.95 : 1.0;
+    for (int k : kChunks) {
+      if (kchunk > 0) k = kchunk;
+      if (kchunk <= 0 && k > cap) break;
+      double groups = 0;
+      for (const StageExtent &b : boxes)
+        groups += double(chl::CeilDiv(b.x, s.tx)) * chl::CeilDiv(b.y, s.ty) * chl::CeilDiv(b.z, std::min(k, b.z));
+      const double rounds = groups <= 4 * slots ? std::ceil(groups / slots) : groups / slots + 0.5;
+      const double cost   = weight * rounds * (k + c0);
+      if (cost < best) best = cost, best_t = t, best_k = k;
+      if (kchunk > 0) break;
+    }
+  }
+  tile = best_t, kchunk = best_k;
+}
+
 int chl_capi::PrepareConfig(chl_hydro_config &c)
 {
-  if (c.tile1 < 0) c.tile1 = 0;
   const bool narrow = c.dual_energy || c.riemann != CHL_RIEMANN_HLLC || c.reconstruction == CHL_RECON_PCM ||
                       c.reconstruction == CHL_RECON_PLMP || c.reconstruction == CHL_RECON_PPMP;  // kernels built for tile shapes 0 and 1 only
-  if (c.tile2 < 0) c.tile2 = narrow ? 0 : 3;
   CHL_TRY(CheckConfig(c));
-  if (c.kchunk1 <= 0) c.kchunk1 = DefaultChunk(c.nz - 2 * c.n_ghost + 2 * (ReconRadius(c.reconstruction) + 1));
-  if (c.kchunk2 <= 0) c.kchunk2 = DefaultChunk(c.nz - 2 * c.n_ghost);
+  const int lx = c.nx - 2 * c.n_ghost, ly = c.ny - 2 * c.n_ghost, lz = c.nz - 2 * c.n_ghost;
+  const int h  = 2 * (ReconRadius(c.reconstruction) + 1);
+  // 1D and 2D boxes do not use them; the shapes only have to be valid
+  const int one = c.ny == 1 || c.nz == 1;
+  const std::vector<StageExtent> s1{one ? StageExtent{1, 1, 1} : StageExtent{lx + h, ly + h, lz + h}};
+  const std::vector<StageExtent> s2{one ? StageExtent{1, 1, 1} : StageExtent{lx, ly, lz}};
+  PickLaunchShape(1, c.precision, c.reconstruction, c.dual_energy != 0, narrow, s1, c.tile1, c.kchunk1);
+  PickLaunchShape(2, c.precision, c.reconstruction, c.dual_energy != 0, narrow, s2, c.tile2, c.kchunk2);
   return CHL_OK;
 }
 

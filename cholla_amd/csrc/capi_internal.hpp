@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <vector>
 
 #include "../../include/cholla_amd.h"
 #include "vl3d_kernels.hpp"
@@ -61,6 +62,14 @@ struct chl_hydro {
 
 namespace chl_capi
 {
+// Cells of one box a stage launch covers, per axis.
+struct StageExtent {
+  int x, y, z;
+};
+// The launch shape of stage 1 or 2 (hydro) over these boxes: tile (kept if >= 0) and z cells
+// per workgroup kchunk (kept if > 0).  narrow: the kernels built for tile shapes 0 and 1 only.
+void PickLaunchShape(int stage, int precision, int reconstruction, bool dual_energy, bool narrow,
+                     const std::vector<StageExtent> &boxes, int &tile, int &kchunk);
 // Fill in the library's defaults (tiles, z-chunks) of a hydro config and check it.
 int PrepareConfig(chl_hydro_config &c);
 // Bytes of the half-step scratch W (and, with dual energy, the pdV sources after w_main).

@@ -1,0 +1,78 @@
+"""The launch shapes the library picks for a box (tile and z planes per workgroup): boxes from
+a few cells to several rounds of workgroups, ragged against every tile, bit-identical to the CPU
+oracle in the reference-order form and to an explicitly shaped launch in the others."""
+import numpy as np
+import pytest
+
+import cholla_amd as chl
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+G = 5 / 3
+
+
+def rough_state(dims, ng, seed, fields=5):
+    """A periodic box of smooth waves with noise on every field (dims: real cells x, y, z)."""
+    nx, ny, nz = (v + 2 * ng for v in dims)
+    rng = np.random.default_rng(seed)
+    z, y, x = np.meshgrid(*[(np.arange(n) - ng + 0.5) / r for n, r in ((nz, dims[2]), (ny, dims[1]), (nx, dims[0]))],
+                          indexing="ij")
+    s = np.sin(2 * np.pi * (x + y)) * np.cos(2 * np.pi * z)
+    d = 1 + 0.3 * s + 0.05 * rng.uniform(-1, 1, s.shape)
+    v = [0.4 * s, 0.3 * np.cos(2 * np.pi * y) + 0 * s, 0.2 * rng.uniform(-1, 1, s.shape)]
+    p = 1 + 0.2 * s
+    U = np.stack([d, d * v[0], d * v[1], d * v[2], p / (G - 1) + 0.5 * d * (v[0] ** 2 + v[1] ** 2 + v[2] ** 2)])
+    U = U.reshape(-1).copy()
+    orc.set_boundaries(U, nx, ny, nz, 5, ng, [1] * 6)
+    return U, (nx, ny, nz)
+
+
+# the smallest periodic box of 4 ghost cells; one plane per workgroup; a remainder in every axis; more than four rounds
+SIZES = [(4, 5, 4), (33, 17, 5), (24, 24, 24), (70, 9, 50), (130, 66, 36)]
+
+
+@pytest.mark.parametrize("recon", [orc.PLMC, orc.PPMC])
+@pytest.mark.parametrize("dims", SIZES)
+def test_picked_shape_matches_oracle(dims, recon):
+    ng = 4
+    U, (nx, ny, nz) = rough_state(dims, ng, 3)
+    w = [1.0 / v for v in dims]
+    A = U.copy()
+    orc.run(A, nx, ny, nz, ng, 5, *w, G, recon, [1] * 6, 0.0, 1e30, 2)
+    D = chl.DeviceArray.from_host(U)
+    hy = chl.Hydro(nx, ny, nz, ng, {orc.PLMC: chl.RECON_PLMC, orc.PPMC: chl.RECON_PPMC}[recon], chl.PREC_FP64_EXACT)
+    hy.run(D, *w, G, 0.0, 1e30, 2)
+    assert np.array_equal(D.download(), A), hy.config().kchunk2
+
+
+@pytest.mark.parametrize("precision", [chl.PREC_FP64, chl.PREC_MIXED])
+@pytest.mark.parametrize("dims", SIZES)
+def test_picked_shape_matches_explicit(dims, precision):
+    ng = 4
+    U, (nx, ny, nz) = rough_state(dims, ng, 4)
+    w = [1.0 / v for v in dims]
+    out = []
+    for kw in ({}, dict(tile1=0, tile2=0, kchunk1=32, kchunk2=32)):
+        D = chl.DeviceArray.from_host(U)
+        hy = chl.Hydro(nx, ny, nz, ng, chl.RECON_PPMC, precision, **kw)
+        hy.run(D, *w, G, 0.0, 1e30, 2)
+        out.append(D.download())
+    # the tiles round alike except where the mixed form's merged lists reorder one sum
+    assert np.abs(out[0] - out[1]).max() <= (0 if precision == chl.PREC_FP64 else 4e-16 * np.abs(out[1]).max())
+
+
+def test_picked_ensemble_shape_matches_single_boxes():
+    ng, dims = 4, [(8, 8, 8), (20, 12, 40), (33, 33, 33)]
+    states, ref = [], []
+    for b, d in enumerate(dims):
+        U, n = rough_state(d, ng, 7 + b)
+        A = U.copy()
+        orc.run(A, *n, ng, 5, *[1.0 / v for v in d], G, orc.PPMC, [1] * 6, 0.0, 1e30, 2)
+        states.append(chl.DeviceArray.from_host(U))
+        ref.append((A, n))
+    ens = chl.Ensemble([n for _, n in ref], ng, chl.RECON_PPMC, chl.PREC_FP64_EXACT)
+    ens.bind(states, [[1.0 / v for v in d] for d in dims])
+    ens.start(G)
+    ens.advance(2)
+    for D, (A, _) in zip(states, ref):
+        assert np.array_equal(D.download(), A)
