@@ -1244,16 +1244,15 @@ __global__ void __launch_bounds__(256, (P::kId == PolicyFast::kId ? 3 : 1)) MhdF
 }
 
 // Stage-2 fluxes along DIR = y or z by a march along DIR: each lane owns a column (x and the
-// third axis) of a 64 x 4 block and walks a chunk of kMarch faces.  Each cell's primitives
+// third axis) of a 64 x 4 block and walks a chunk of march faces.  Each cell's primitives
 // (Load_Data) are recovered once and slide through the reconstruction stencil's window, each
 // cell is reconstructed once, and its face-(i+1/2) state carries to the next face: a chunk of
 // K faces loads K + 2 R cells and reconstructs K + 1 (a 64 x 4 face tile across DIR would
 // reconstruct 5 rows for 4, and each reconstruction recovers its 2 R + 1 cells' primitives).
 // Each face's flux is the tile kernel's: HLLD of the two cells' interface states, stored at
 // the lower cell.
-constexpr int kMarch = 16;
 template <class P, int DIR, int RK = 1>
-__global__ void __launch_bounds__(256) MhdFlux2MarchKernel(MhdArgs a, int lo, int hix, int hiy, int hiz)
+__global__ void __launch_bounds__(256) MhdFlux2MarchKernel(MhdArgs a, int lo, int hix, int hiy, int hiz, int march)
 {
   static_assert(DIR == 1 || DIR == 2, "the x faces use MhdFlux2TileKernel");
   using T = typename P::T;
@@ -1263,11 +1262,11 @@ __global__ void __launch_bounds__(256) MhdFlux2MarchKernel(MhdArgs a, int lo, in
   const int his = DIR == 2 ? hiz : hiy, hit = DIR == 2 ? hiy : hiz;  // march axis and third axis bounds
   const int tx = threadIdx.x % 64, tt = threadIdx.x / 64;
   // blocks in XCD-contiguous order: x fastest, then the third axis, then the chunk along DIR
-  const int gx = (hix - lo + 64) / 64, gt = (hit - lo + 4) / 4, gs = (his - lo + kMarch) / kMarch;
+  const int gx = (hix - lo + 64) / 64, gt = (hit - lo + 4) / 4, gs = (his - lo + march) / march;
   const int q = XcdItem(int(blockIdx.x), gx * gt * gs);
   if (q >= gx * gt * gs) return;
   const int x = lo + (q % gx) * 64 + tx, t = lo + ((q / gx) % gt) * 4 + tt;
-  const int s0 = lo + (q / (gx * gt)) * kMarch, s1 = min(s0 + kMarch - 1, his);
+  const int s0 = lo + (q / (gx * gt)) * march, s1 = min(s0 + march - 1, his);
   if (x > hix || t > hit) return;  // no barrier below
   const double *Uh = a.Uh;
   const T g        = T(a.gamma);
