@@ -1,0 +1,33 @@
+"""The snapshot transposes at the edges of their 64 x 32 tiles, against the numpy transpose."""
+import numpy as np
+import pytest
+
+import cholla_amd as chl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("direction", [-1, 0, 1, 2])
+@pytest.mark.parametrize("dims", [(1, 2, 1), (63, 3, 31), (64, 2, 32), (65, 5, 33), (9, 1, 130), (200, 7, 4)])
+def test_pack_and_unpack_tiles(dims, direction):
+    nxr, nyr, nzr = dims
+    ng = 3
+    nx, ny, nz = nxr + 2 * ng, nyr + 2 * ng, nzr + 2 * ng
+    ext = [n + (direction == a) for a, n in enumerate(dims)]
+    lo = [ng - (direction == a) for a in range(3)]
+    rng = np.random.default_rng(1)
+    F = rng.normal(size=(nz, ny, nx))
+    want = F[lo[2]:lo[2] + ext[2], lo[1]:lo[1] + ext[1], lo[0]:lo[0] + ext[0]].transpose(2, 1, 0)
+    D, buf = chl.DeviceArray.from_host(F), chl.DeviceArray(want.size, np.full(want.size, -7.0))
+    args = (nx, ny, nz, ng, *ext, direction)
+    chl.check(chl.lib().chl_pack_real_cells(D.ptr, buf.ptr, *args))
+    assert np.array_equal(buf.download().reshape(want.shape), want)
+    b32 = chl.DeviceArray(want.size, np.zeros(want.size))
+    chl.check(chl.lib().chl_pack_real_cells_f32(D.ptr, b32.ptr, *args))
+    assert np.array_equal(b32.download().view(np.float32)[:want.size].reshape(want.shape), want.astype(np.float32))
+    G0 = rng.normal(size=F.shape)
+    G = chl.DeviceArray.from_host(G0)
+    chl.check(chl.lib().chl_unpack_real_cells(buf.ptr, G.ptr, *args))
+    out = G0.copy()
+    out[lo[2]:lo[2] + ext[2], lo[1]:lo[1] + ext[1], lo[0]:lo[0] + ext[0]] = want.transpose(2, 1, 0)
+    assert np.array_equal(G.download().reshape(F.shape), out)
