@@ -3,7 +3,7 @@
     python -m cholla_amd.build        # or cholla_amd.build.build()
 
 Every HIP translation unit is compiled for gfx950 with packed-FP32 instructions
-disabled.  The FP64 reference-order kernels (hydro_exact.hip, support_kernels.hip,
+disabled.  The FP64 reference-order kernels (hydro_exact.hip, support_kernels.hip, vl_small.hip,
 ensemble_exact.hip, mhd_exact.hip) are built with -ffp-contract=off.  The fast FP64
 and mixed-precision kernels (hydro_fast.hip, ensemble_fast.hip, mhd_fast.hip) are
 built with -ffp-contract=on: a product and a sum are fused only where they sit in
@@ -34,6 +34,7 @@ COMMON = [
 UNITS = [
     ("hydro_exact.hip", ["-ffp-contract=off"]),
     ("support_kernels.hip", ["-ffp-contract=off"]),
+    ("vl_small.hip", ["-ffp-contract=off"]),
     ("snapshot_kernels.hip", ["-ffp-contract=off"]),
     ("hydro_fast.hip", ["-ffp-contract=on"]),
     ("ensemble_exact.hip", ["-ffp-contract=off"]),

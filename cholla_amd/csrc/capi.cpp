@@ -192,6 +192,16 @@ int EnqueueStep(chl_hydro *h, double *U, double dx, double dy, double dz, double
     return CHL_OK;
   }
   if (h->two_d) {  // no temperature floor: the reference's guard admits no 2D cell (hydro_cuda.cu:1130-1131)
+    if (chl::Vl2dFusedTakes(c.ny, c.reconstruction, SolverKind(c.riemann), c.dual_energy != 0, h->grav)) {
+      bool images = fill && c.nx >= 3 * ng && c.ny >= 3 * ng;
+      for (int q = 0; q < 4; q++) images = images && c.bc_flags[q] == CHL_BC_PERIODIC;
+      CHL_HIP(chl::LaunchVl2dFused(U, reinterpret_cast<double *>(h->W), c.nx, c.ny, ng, c.reconstruction, c.precision,
+                                   dx, dy, dt_dev, dt_host, gamma, images, update_grid ? h->dti() : nullptr,
+                                   h->stream));
+      if (fill && !images)
+        CHL_HIP(chl::LaunchGhostFill(U, c.nx, c.ny, c.nz, c.n_fields, ng, c.bc_flags, h->stream));
+      return CHL_OK;
+    }
     CHL_HIP(chl::LaunchVl2d(U, reinterpret_cast<double *>(h->W), c.nx, c.ny, ng, c.reconstruction,
                             SolverKind(c.riemann), c.dual_energy != 0, c.precision, dx, dy, dt_dev, dt_host, gamma,
                             update_grid ? h->dti() : nullptr, h->grav, h->stream));
@@ -293,6 +303,22 @@ int EnsureGraph(chl_hydro *h, double *U, double dx, double dy, double dz, double
   CHL_HIP(e3);
   h->g_U = U;
   std::memcpy(h->g_key, key, sizeof(key));
+  return CHL_OK;
+}
+
+// A small 1D box runs whole batches of device-timed steps in one launch.
+bool OneLaunchRun(const chl_hydro *h)
+{
+  const chl_hydro_config &c = h->cfg;
+  return h->one_d && chl::Vl1dRunTakes(c.nx, c.reconstruction, SolverKind(c.riemann), c.dual_energy != 0, h->grav);
+}
+
+int EnqueueRun1d(chl_hydro *h, double *U, double dx, double gamma, int n_steps, bool first, double t0, double tout)
+{
+  const chl_hydro_config &c = h->cfg;
+  static_assert(sizeof(chl::LineClock) == 32, "the layout of the handle's device scalars");
+  CHL_HIP(chl::LaunchVl1dRun(U, c.nx, c.n_ghost, c.reconstruction, c.precision, dx, gamma, c.bc_flags, n_steps, first,
+                             t0, tout, kCfl, reinterpret_cast<chl::LineClock *>(h->scal), h->stream));
   return CHL_OK;
 }
 
@@ -554,6 +580,19 @@ int chl_hydro_run(chl_hydro *h, double *U, double dx, double dy, double dz, doub
                   double U_floor, double t0, double tout, int max_steps, int use_graph, double *t_out, int *steps_out)
 {
   if (!h || !U) return Fail(CHL_ERR_INVALID, "null argument");
+  if (OneLaunchRun(h)) {
+    chl::LineClock k{0, 0.0, t0, 0};
+    for (int done = 0; done < max_steps && k.t < tout;) {
+      const int batch = std::min(1024, max_steps - done);
+      CHL_TRY(EnqueueRun1d(h, U, dx, gamma, batch, done == 0, t0, tout));
+      CHL_HIP(hipMemcpyAsync(&k, h->scal, sizeof(k), hipMemcpyDeviceToHost, h->stream));
+      CHL_HIP(hipStreamSynchronize(h->stream));
+      done += batch;
+    }
+    if (t_out) *t_out = k.t;
+    if (steps_out) *steps_out = k.nstep;
+    return CHL_OK;
+  }
   CHL_TRY(InitialDti(h, U, dx, dy, dz, gamma));
   CHL_TRY(SetTimeState(h, t0));
   if (use_graph) CHL_TRY(EnsureGraph(h, U, dx, dy, dz, gamma, density_floor, U_floor, tout));
@@ -584,16 +623,21 @@ int chl_hydro_time_steps(chl_hydro *h, double *U, double dx, double dy, double d
                          int use_graph, float *ms_out, double *dt_last_out)
 {
   if (!h || !U || n_steps < 0) return Fail(CHL_ERR_INVALID, "bad argument");
-  const double tout = std::numeric_limits<double>::infinity();
-  CHL_TRY(InitialDti(h, U, dx, dy, dz, gamma));
-  CHL_TRY(SetTimeState(h, 0.0));
-  if (use_graph) CHL_TRY(EnsureGraph(h, U, dx, dy, dz, gamma, 0.0, 0.0, tout));
+  const double tout     = std::numeric_limits<double>::infinity();
+  const bool one_launch = OneLaunchRun(h);
+  if (!one_launch) {
+    CHL_TRY(InitialDti(h, U, dx, dy, dz, gamma));
+    CHL_TRY(SetTimeState(h, 0.0));
+    if (use_graph) CHL_TRY(EnsureGraph(h, U, dx, dy, dz, gamma, 0.0, 0.0, tout));
+  }
   hipEvent_t e0, e1;
   CHL_HIP(hipEventCreate(&e0));
   CHL_HIP(hipEventCreate(&e1));
   CHL_HIP(hipStreamSynchronize(h->stream));
   CHL_HIP(hipEventRecord(e0, h->stream));
-  for (int s = 0; s < n_steps; s++) {
+  for (int s = 0; one_launch && s < n_steps; s += 1024)
+    CHL_TRY(EnqueueRun1d(h, U, dx, gamma, std::min(1024, n_steps - s), s == 0, 0.0, tout));
+  for (int s = 0; !one_launch && s < n_steps; s++) {
     if (use_graph) {
       CHL_HIP(hipGraphLaunch(h->graph, h->stream));
     } else {

@@ -45,6 +45,21 @@ hipError_t LaunchVl1d(double *U, double *W, int n, int ng, int recon, int rieman
 hipError_t LaunchVl2d(double *U, double *scratch, int nx, int ny, int ng, int recon, int riemann, bool de, int form,
                       double dx, double dy, const double *dt_dev, double dt, double gamma, unsigned long long *dti,
                       const GravSpec &grav, hipStream_t s);
+// A batch of 1D steps in one launch, and the fused 2D step (vl_small.hip).  *Takes: whether the
+// options are ones these kernels are compiled for.  first: start the clock at t0 with the
+// state's own inverse dt, else go on from *clk, which holds the device scalars of a handle.
+struct LineClock {
+  unsigned long long dti;
+  double dt, t;
+  int nstep;
+};
+bool Vl1dRunTakes(int n, int recon, int riemann, bool de, const GravSpec &grav);
+hipError_t LaunchVl1dRun(double *U, int n, int ng, int recon, int form, double dx, double gamma, const int flags[6],
+                         int n_steps, bool first, double t0, double tout, double cfl, LineClock *clk, hipStream_t s);
+bool Vl2dFusedTakes(int ny, int recon, int riemann, bool de, const GravSpec &grav);
+hipError_t LaunchVl2dFused(double *U, double *W, int nx, int ny, int ng, int recon, int form, double dx, double dy,
+                           const double *dt_dev, double dt, double gamma, bool periodic, unsigned long long *dti,
+                           hipStream_t s);
 hipError_t LaunchReconGrid(int recon, const double *U, double *QL, double *QR, int nx, int ny, int nz, double gamma,
                            int dir, hipStream_t s);
 hipError_t LaunchRiemannGrid(int riemann, const double *QL, const double *QR, double *F, int nx, int ny, int nz,
