@@ -102,3 +102,23 @@ def test_mhd_chunks_match_oracle(dims, recon, ng):
                 reconstruction={orc.MHD_PLMC: chl.RECON_PLMC, orc.MHD_PPMC: chl.RECON_PPMC}[recon])
     h.run(D, *w, G, 0.0, 1e30, 2)
     assert np.isfinite(A).all() and np.array_equal(D.download(), A)
+
+
+@pytest.mark.parametrize("dims", [(4, 5, 4), (65, 5, 9), (63, 33, 17), (96, 40, 44)])
+def test_de_sync_columns_match_oracle(dims):
+    # columns of 64 x 4 with remainders in x and y, one workgroup, one and several planes each
+    ng = 4
+    U5, (nx, ny, nz) = rough_state(dims, ng, 11)
+    U = np.concatenate([U5, np.zeros(nx * ny * nz)])
+    a = U.reshape(6, -1)
+    a[5] = a[4] - 0.5 * (a[1] ** 2 + a[2] ** 2 + a[3] ** 2) / a[0]
+    a[1] += 100.0 * a[0] * (np.arange(a[0].size) // nx % ny < ny // 2)  # a hypersonic slab: both sides of the switch
+    a[4] = a[5] + 0.5 * (a[1] ** 2 + a[2] ** 2 + a[3] ** 2) / a[0]
+    orc.set_boundaries(U, nx, ny, nz, 6, ng, [1] * 6)
+    w = [1.0 / v for v in dims]
+    A = U.copy()
+    _, t = orc.run(A, nx, ny, nz, ng, 6, *w, G, orc.PLMC, [1] * 6, 0.0, 1e30, 2, dual_energy_on=True)
+    D = chl.DeviceArray.from_host(U)
+    hy = chl.Hydro(nx, ny, nz, ng, chl.RECON_PLMC, chl.PREC_FP64_EXACT, dual_energy=True)
+    _, tg = hy.run(D, *w, G, 0.0, 1e30, 2)
+    assert np.isfinite(A).all() and tg == t and np.array_equal(D.download(), A)
