@@ -270,13 +270,14 @@ __device__ __forceinline__ void FluxGlobal(const Cons<typename P::T> &f, typenam
 
 // The Riemann solve (HLLC, or HLL under an HllPolicy) on one face; the flux in global
 // component order into out[0..4] and, with dual energy, the GasEnergy flux into out[5].
-template <class P, int DIR, bool DE>
+// HALF: a face of the half step (see Hllc).
+template <class P, int DIR, bool DE, bool HALF = false>
 __device__ __forceinline__ void FaceFlux(const RState<typename P::T> &l, const RState<typename P::T> &r,
                                          typename P::T gamma, typename P::T *out)
 {
   using T = typename P::T;
   T fge   = T(0);
-  Cons<T> f = RiemannFlux<P, DE>(l, r, gamma, &fge);
+  Cons<T> f = RiemannFlux<P, DE, HALF>(l, r, gamma, &fge);
   FluxGlobal<P, DIR>(f, out);
   if constexpr (DE) out[kGasEnergy] = fge;
 }
@@ -295,7 +296,7 @@ __device__ __forceinline__ void PcmFaceFlux(const PcmCell<typename P::T, DE> &a,
     l.pd        = a.plo;
     r.pd        = (b.p - a.p) + b.plo;
   }
-  FaceFlux<P, DIR, DE>(l, r, gamma, out);
+  FaceFlux<P, DIR, DE, true>(l, r, gamma, out);
 }
 
 // Dual energy: the DE pressure of a cell and its centred velocity-difference source

@@ -76,14 +76,14 @@ __device__ __forceinline__ RState<typename P::T> SideFromCons(double d, double m
 }
 
 // The flux of one face in FP64 from its two Riemann inputs (the split pressure's p0 added
-// back to the normal-momentum flux); fge the GasEnergy flux under DE.
-template <class P, bool DE>
+// back to the normal-momentum flux); fge the GasEnergy flux under DE, HALF as in Hllc.
+template <class P, bool DE, bool HALF = false>
 __device__ __forceinline__ Cons<double> FluxFp64(const RState<typename P::T> &l, const RState<typename P::T> &r,
                                                  typename P::T gamma, double *fge)
 {
   using T = typename P::T;
   T g     = T(0);
-  const Cons<T> f = RiemannFlux<P, DE>(l, r, gamma, &g);
+  const Cons<T> f = RiemannFlux<P, DE, HALF>(l, r, gamma, &g);
   Cons<double> o{double(f.d), double(f.mx), double(f.my), double(f.mz), double(f.E)};
   if constexpr (SplitPressure<P>) o.mx += double(l.p0);
   *fge = double(g);
@@ -102,7 +102,7 @@ __device__ __forceinline__ Cons<double> PcmFlux(RState<typename P::T> a, double 
     b.pd        = (b.p - a.p) + T(blo);
     a.pd        = T(alo);
   }
-  return FluxFp64<P, DE>(a, b, gamma, fge);
+  return FluxFp64<P, DE, true>(a, b, gamma, fge);
 }
 
 // The interface values of the centre cell of a stencil of FP64 primitives w (in the sweep's
