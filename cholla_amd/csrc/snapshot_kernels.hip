@@ -5,14 +5,14 @@
 // real cells is z-fastest, buf = k + j*nz_real + i*nz_real*ny_real (CopyReal3D_GPU_Kernel,
 // src/io/io_gpu.cu:44-60; Fill_HDF5_Buffer_From_Grid_CPU and Fill_Grid_From_HDF5_Buffer,
 // src/io/io.cpp:1232-1268 and 2450-2490).  Between the two the fastest index changes from x
-// to z, so each workgroup moves a 64 (x) by 32 (z) tile of one y row through LDS: the grid
-// side reads (or writes) rows of 64 consecutive x and the snapshot side writes (or reads) rows
-// of 32 consecutive z.  Bound by HBM: 16 bytes per cell.  Grid rows start n_ghost cells into a
-// line, so neighbouring tiles share a line at each row end; the tiles go out in XCD-contiguous
-// order, x fastest, which keeps both halves of that line in one L2 (two XCDs each fetched it,
-// or wrote its half through).  A 256^3 field: unpack 84.7 -> 61.9 us, pack 54.7 -> 54.8;
-// 300x212x190: pack 57.8 -> 42.4 us, unpack 56.4 -> 44.0 (4.3-4.9 TB/s; a plain copy reaches
-// 4.8), against 32x32 tiles in dispatch order.
+// to z, so each workgroup moves a tile of one y row through LDS, 64 (x) by 32 (z) or 32 by 32:
+// the grid side reads (or writes) rows of consecutive x and the snapshot side writes (or reads)
+// rows of 32 consecutive z.  Bound by HBM on large fields: 16 bytes per cell.  Grid rows start
+// n_ghost cells into a line, so neighbouring tiles share a line at each row end; the 64 x 32
+// tiles go out in XCD-contiguous order, x fastest, which keeps both halves of that line in one
+// L2 (two XCDs each fetched it, or wrote its half through).  A 256^3 field: unpack 84.7 -> 61.9
+// us, pack 54.7 -> 54.8; 300x212x190: pack 57.8 -> 42.4 us, unpack 56.4 -> 44.0 (4.3-4.9 TB/s;
+// a plain copy reaches 4.8), against 32x32 tiles in dispatch order.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
@@ -24,21 +24,27 @@ namespace chl
 namespace
 {
 
-constexpr int kTX = 64, kTZ = 32;  // tile: x by z
+constexpr int kTZ = 32;  // tile: TX by kTZ, x by z
 constexpr int kThreads = 256;
 
 // PACK: grid -> buf (converted to OUT); !PACK: buf -> grid.  (ox, oy, oz) is the grid index of
 // the dataset's first element: n_ghost, or n_ghost - 1 along a magnetic field's own axis
-// (its dataset holds one more face than there are real cells).
-template <bool PACK, typename OUT>
+// (its dataset holds one more face than there are real cells).  TX 64: a linear grid of
+// tiles in XCD-contiguous order; TX 32: the grid's axes are the tiles'.
+template <bool PACK, typename OUT, int kTX>
 __global__ void __launch_bounds__(kThreads) SnapshotTileKernel(double *grid, OUT *buf, int nx, int ny, int nxr, int nyr,
-                                                              int nzr, int ox, int oy, int oz, int gx, int gz,
-                                                              long tiles)
+                                                              int nzr, int ox, int oy, int oz, unsigned gx,
+                                                              unsigned gz, unsigned tiles)
 {
   __shared__ double t[kTZ][kTX + 1];
-  const long per = (tiles + 7) / 8, q = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if ((blockIdx.x >> 3) >= per || q >= tiles) return;
-  const int i0 = int(q % gx) * kTX, k0 = int(q / gx % gz) * kTZ, j = int(q / (long(gx) * gz));
+  int i0, k0, j;
+  if constexpr (kTX == 64) {
+    const unsigned per = (tiles + 7) / 8, q = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((blockIdx.x >> 3) >= per || q >= tiles) return;
+    i0 = int(q % gx) * kTX, k0 = int(q / gx % gz) * kTZ, j = int(q / (gx * gz));
+  } else {
+    i0 = int(blockIdx.x) * kTX, k0 = int(blockIdx.y) * kTZ, j = int(blockIdx.z);
+  }
   const size_t plane = size_t(nx) * ny;
   auto gid = [&](int i, int k) { return size_t(i + ox) + size_t(j + oy) * nx + size_t(k + oz) * plane; };
   auto bid = [&](int i, int k) { return size_t(k) + size_t(j) * nzr + size_t(i) * nzr * nyr; };
@@ -71,13 +77,24 @@ __global__ void __launch_bounds__(kThreads) SnapshotTileKernel(double *grid, OUT
   }
 }
 
+// From this many cells the tiles are 64 x 32 in XCD-contiguous order.  Below it a field and its
+// buffer stay in the caches, lines shared by two XCDs cost little and more, smaller workgroups
+// start sooner: 10 transposes and their launches of 80^3 take 166 us in 32 x 32 tiles against
+// 182, 160^3 308 against 313, 200^3 456 against 454, 256^3 841 against 748.
+constexpr size_t kLargeField = size_t(8) << 20;
+
 template <bool PACK, typename OUT>
 hipError_t Launch(double *grid, OUT *buf, const SnapshotShape &s, hipStream_t st)
 {
-  const int gx = (s.nxr + kTX - 1) / kTX, gz = (s.nzr + kTZ - 1) / kTZ;
-  const long tiles = long(gx) * gz * s.nyr;
-  hipLaunchKernelGGL((SnapshotTileKernel<PACK, OUT>), dim3(unsigned((tiles + 7) / 8 * 8)), dim3(kThreads), 0, st, grid,
-                     buf, s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, gx, gz, tiles);
+  const unsigned gz = unsigned((s.nzr + kTZ - 1) / kTZ);
+  if (size_t(s.nxr) * s.nyr * s.nzr < kLargeField && s.nyr <= 65535) {
+    hipLaunchKernelGGL((SnapshotTileKernel<PACK, OUT, 32>), dim3(unsigned((s.nxr + 31) / 32), gz, unsigned(s.nyr)),
+                       dim3(kThreads), 0, st, grid, buf, s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, 0u, 0u, 0u);
+    return hipGetLastError();
+  }
+  const unsigned gx = unsigned((s.nxr + 63) / 64), tiles = gx * gz * unsigned(s.nyr);
+  hipLaunchKernelGGL((SnapshotTileKernel<PACK, OUT, 64>), dim3((tiles + 7) / 8 * 8), dim3(kThreads), 0, st, grid, buf,
+                     s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, gx, gz, tiles);
   return hipGetLastError();
 }
 

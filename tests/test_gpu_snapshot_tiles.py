@@ -1,4 +1,5 @@
-"""The snapshot transposes at the edges of their 64 x 32 tiles, against the numpy transpose."""
+"""The snapshot transposes at the edges of their tiles (32 x 32, and 64 x 32 from 2^23 cells on),
+against the numpy transpose."""
 import numpy as np
 import pytest
 
@@ -31,3 +32,18 @@ def test_pack_and_unpack_tiles(dims, direction):
     out = G0.copy()
     out[lo[2]:lo[2] + ext[2], lo[1]:lo[1] + ext[1], lo[0]:lo[0] + ext[0]] = want.transpose(2, 1, 0)
     assert np.array_equal(G.download().reshape(F.shape), out)
+
+
+@pytest.mark.parametrize("dims", [(65, 3, 43019), (8388607, 1, 1), (129, 2033, 32), (64, 4096, 33)])
+def test_pack_and_unpack_large_fields(dims):
+    # just below and above the size where the tiles change, with remainders in x and z
+    rng = np.random.default_rng(2)
+    F = rng.normal(size=dims[::-1])
+    want = F.transpose(2, 1, 0)
+    D, buf = chl.DeviceArray.from_host(F), chl.DeviceArray(F.size, np.zeros(F.size))
+    args = (*dims, 0, *dims, -1)
+    chl.check(chl.lib().chl_pack_real_cells(D.ptr, buf.ptr, *args))
+    assert np.array_equal(buf.download().reshape(want.shape), want)
+    G = chl.DeviceArray(F.size, np.zeros(F.size))
+    chl.check(chl.lib().chl_unpack_real_cells(buf.ptr, G.ptr, *args))
+    assert np.array_equal(G.download().reshape(F.shape), F)
