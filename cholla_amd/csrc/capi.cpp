@@ -171,12 +171,30 @@ int LaunchDualEnergy(chl_hydro *h, const chl::StepArgs &a)
   return CHL_OK;
 }
 
+// What a 3D step starts with: the side buffer of its repairs (a.rep.side) and, with tout, the
+// device clock, in one launch where there are both.
+int LaunchStepStart(chl_hydro *h, const chl::StepArgs &a, const double *tout)
+{
+  if (a.rep.side) {
+    const chl::StepClock clk =
+        tout ? chl::StepClock{h->dti(), h->dt(), h->t(), *tout, kCfl, h->nstep()} : chl::StepClock{};
+    CHL_HIP(chl::LaunchRepairSide(a, clk, h->stream));
+  } else if (tout) {
+    CHL_HIP(chl::LaunchDtAdvance(h->dti(), h->dt(), h->t(), *tout, kCfl, h->nstep(), h->stream));
+  }
+  return CHL_OK;
+}
+
 // Enqueue one VL step.  mode: 0 = VL only, 1 = VL + floors + dti, (fill) ghost refresh.
+// tout: not null advances the device clock first, up to *tout.
 int EnqueueStep(chl_hydro *h, double *U, double dx, double dy, double dz, double gamma, double dt_host,
-                const double *dt_dev, double density_floor, double U_floor, bool update_grid, bool fill)
+                const double *dt_dev, double density_floor, double U_floor, bool update_grid, bool fill,
+                const double *tout = nullptr)
 {
   const chl_hydro_config &c = h->cfg;
   const int ng              = c.n_ghost;
+  if (tout && (h->one_d || h->two_d))
+    CHL_HIP(chl::LaunchDtAdvance(h->dti(), h->dt(), h->t(), *tout, kCfl, h->nstep(), h->stream));
   if (h->one_d) {
     const int n = c.nx;
     // the dt reduction rides on the last kernel of the step: the one-block stage 2, or with
@@ -228,7 +246,7 @@ int EnqueueStep(chl_hydro *h, double *U, double dx, double dy, double dz, double
   // stage 2 overwrites ghost cells with new periodic images: a density repair next to one
   // reads the pre-step value from the side buffer instead
   if (!(fused_ghosts && c.density_floor && !c.dual_energy)) a.rep.side = nullptr;
-  if (a.rep.side) CHL_HIP(chl::LaunchRepairSide(a, h->stream));
+  CHL_TRY(LaunchStepStart(h, a, tout));
   CHL_TRY(LaunchStage1(h, a));
   CHL_TRY(LaunchStage2(h, a));
   CHL_HIP(c.precision == CHL_PREC_FP64_EXACT ? chl::LaunchRepairExact(a, h->stream)
@@ -279,8 +297,7 @@ int SetTimeState(chl_hydro *h, double t0)
 int EnqueueDeviceStep(chl_hydro *h, double *U, double dx, double dy, double dz, double gamma, double density_floor,
                       double U_floor, double tout)
 {
-  CHL_HIP(chl::LaunchDtAdvance(h->dti(), h->dt(), h->t(), tout, kCfl, h->nstep(), h->stream));
-  return EnqueueStep(h, U, dx, dy, dz, gamma, 0.0, h->dt(), density_floor, U_floor, true, true);
+  return EnqueueStep(h, U, dx, dy, dz, gamma, 0.0, h->dt(), density_floor, U_floor, true, true, &tout);
 }
 
 int EnsureGraph(chl_hydro *h, double *U, double dx, double dy, double dz, double gamma, double density_floor,
@@ -677,8 +694,7 @@ int chl_hydro_kernel_times(chl_hydro *h, double *U, double dx, double dy, double
   if (!(fused_ghosts && c.density_floor && !c.dual_energy)) a.rep.side = nullptr;
   for (int s = 0; s < n_steps; s++) {
     CHL_HIP(hipEventRecord(ev[0], h->stream));
-    CHL_HIP(chl::LaunchDtAdvance(h->dti(), h->dt(), h->t(), tout, kCfl, h->nstep(), h->stream));
-    if (a.rep.side) CHL_HIP(chl::LaunchRepairSide(a, h->stream));
+    CHL_TRY(LaunchStepStart(h, a, &tout));
     CHL_HIP(hipEventRecord(ev[1], h->stream));
     CHL_TRY(LaunchStage1(h, a));
     CHL_HIP(hipEventRecord(ev[2], h->stream));

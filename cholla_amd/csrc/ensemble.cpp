@@ -572,7 +572,6 @@ int chl_ensemble_advance_looped(chl_ensemble *e, int n_steps, float *ms_out)
       for (int b : e->order) {
         const chl::BoxDesc &d = e->hbox[b];
         chl::BoxClock *k      = e->clk + b;
-        CHL_HIP(chl::LaunchDtAdvance(&k->dti, &k->dt, &k->t, d.tout, kCfl, &k->nstep, e->stream));
         chl::StepArgs a{};
         a.U = d.U, a.W = d.W, a.pdv = d.pdv, a.nx = d.nx, a.ny = d.ny, a.nz = d.nz, a.ng = c.n_ghost;
         a.dx = d.dx, a.dy = d.dy, a.dz = d.dz, a.gamma = e->gamma, a.dt = 0.0, a.dt_dev = &k->dt, a.dti = &k->dti;
@@ -582,7 +581,11 @@ int chl_ensemble_advance_looped(chl_ensemble *e, int n_steps, float *ms_out)
         a.riemann = c.riemann;
         a.rep    = d.rep;
         a.kchunk = d.kchunk1;
-        if (a.rep.side) CHL_HIP(chl::LaunchRepairSide(a, e->stream));
+        if (a.rep.side) {
+          CHL_HIP(chl::LaunchRepairSide(a, {&k->dti, &k->dt, &k->t, d.tout, kCfl, &k->nstep}, e->stream));
+        } else {
+          CHL_HIP(chl::LaunchDtAdvance(&k->dti, &k->dt, &k->t, d.tout, kCfl, &k->nstep, e->stream));
+        }
         CHL_HIP(pol == CHL_PREC_FP64_EXACT ? chl::LaunchStage1Exact(a, R1, c.tile1, e->stream)
                                            : chl::LaunchStage1Fast(pol, a, R1, c.tile1, e->stream));
         a.kchunk = d.kchunk2;

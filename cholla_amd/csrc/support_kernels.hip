@@ -311,14 +311,7 @@ __global__ void DtAdvanceKernel(unsigned long long *dti_bits, double *dt_dev, do
                                 double cfl, int *n_step, int take)
 {
   const unsigned long long bits = take ? atomicExch(dti_bits, 0ull) : *dti_bits;
-  double dti = __longlong_as_double((long long)bits);
-  double t   = *t_dev;
-  double dt  = cfl / dti;
-  if (t + dt > tout) dt = tout - t;
-  if (!(t < tout)) dt = 0.0;
-  *dt_dev = dt;
-  *t_dev  = t + dt;
-  if (dt > 0.0) *n_step += 1;
+  AdvanceClock(__longlong_as_double((long long)bits), dt_dev, t_dev, tout, cfl, n_step);
 }
 
 // One thread per box: the same dt and clock arithmetic as DtAdvanceKernel, then the

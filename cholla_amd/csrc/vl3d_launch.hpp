@@ -169,7 +169,14 @@ hipError_t LaunchRepair(const StepArgs &a, hipStream_t s)
 }
 
 // The side buffer of a density repair next to fused periodic images (hydro_exact.hip).
-hipError_t LaunchRepairSide(const StepArgs &a, hipStream_t s);
+// The device scalars of a step's clock (AdvanceClock); dti null: none.
+struct StepClock {
+  const unsigned long long *dti;
+  double *dt, *t, tout, cfl;
+  int *nstep;
+};
+// The side buffer of a.rep, and with clk.dti the clock of the step.
+hipError_t LaunchRepairSide(const StepArgs &a, const StepClock &clk, hipStream_t s);
 
 // Explicitly instantiated per policy in hydro_exact.hip / hydro_fast.hip.
 hipError_t LaunchStage1Policy(int policy, const StepArgs &a, int R1, int tile, hipStream_t s);
