@@ -393,7 +393,10 @@ size_t chl_capi::HalfStepBytes(const chl_hydro_config &c, size_t *w_main)
 // worst; the 32-plane chunks of one fixed tile it replaced left a 48^3 box to 12-18 workgroups
 // (stage 1 / 2, PLMC, reference order: 209 / 406 us against 22 / 34) and KH 512^3 (mixed) on
 // stage-2 tiles of 16x8 (10.2 ms against 8.5).
-//   tiles    stage 1: 16x16 (FP64), 32x8 (mixed: KH 256^3 495 against 536 us); stage 2: 16x16,
+//   tiles    stage 1: 16x16 (FP64), 32x8 (mixed: KH 256^3 495 against 536 us), or 64x4 where
+//            its wider rows fit the box (mixed: 300x212x190 289 against 326 us, 512^3 3.12
+//            against 3.30 ms; 200x180x160, a quarter of whose lanes it would idle, 173 against
+//            169 us), which the narrow kernels do not have; stage 2: 16x16,
 //            and 32x16 in the FP64 forms where it rounds better (with PLMC it needs 5 % less:
 //            KH 256^3 1.89 against 2.09 ms), or 16x8 where those leave CUs idle (32^3, PPMC,
 //            fast form: 27 against 28 us), which the narrow kernels do not have
@@ -408,7 +411,8 @@ void chl_capi::PickLaunchShape(int stage, int precision, int reconstruction, boo
   const int cap    = stage == 1 ? (mixed ? 16 : 8) : (dual_energy ? 8 : 32);
   const double c0  = stage == 1 ? 1.0 : 0.5;
   const bool all   = stage == 2 && !mixed && !narrow;
-  int tiles[3]     = {stage == 1 && mixed ? 0 : 1, all ? 3 : -1, all ? 4 : -1};
+  const bool wide  = stage == 1 && mixed && !narrow;
+  int tiles[3]     = {stage == 1 && mixed ? 0 : 1, all ? 3 : (wide ? 2 : -1), all ? 4 : -1};
   if (all) std::swap(tiles[0], tiles[1]);  // equal costs: the first
   if (tile >= 0) tiles[0] = tile, tiles[1] = tiles[2] = -1;
   static const int kChunks[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32};
@@ -418,7 +422,7 @@ void chl_capi::PickLaunchShape(int stage, int precision, int reconstruction, boo
     if (t < 0 || t >= chl::kNumTiles) continue;
     const chl::TileShape s = chl::kTiles[t];
     const double slots     = t == 3 && tile < 0 ? cus : double(cus) * std::max(1, 4 * waves * 64 / (s.tx * s.ty));
-    const double weight    = t == 4 && reconstruction == CHL_RECON_PLMC ? 0.95 : 1.0;
+    const double weight    = t == 4 && reconstruction == CHL_RECON_PLMC ? 0.95 : (wide && t == 2 ? 0.93 : 1.0);
     for (int k : kChunks) {
       if (kchunk > 0) k = kchunk;
       if (kchunk <= 0 && k > cap) break;

@@ -122,3 +122,18 @@ def test_de_sync_columns_match_oracle(dims):
     hy = chl.Hydro(nx, ny, nz, ng, chl.RECON_PLMC, chl.PREC_FP64_EXACT, dual_energy=True)
     _, tg = hy.run(D, *w, G, 0.0, 1e30, 2)
     assert np.isfinite(A).all() and tg == t and np.array_equal(D.download(), A)
+
+
+@pytest.mark.parametrize("dims,wide", [((122, 40, 20), True), ((250, 34, 9), True), ((130, 66, 36), False)])
+def test_mixed_stage1_wide_tiles(dims, wide):
+    ng = 4
+    U, (nx, ny, nz) = rough_state(dims, ng, 6)
+    w = [1.0 / v for v in dims]
+    out = []
+    for kw in ({}, dict(tile1=0, kchunk1=32)):
+        D = chl.DeviceArray.from_host(U)
+        hy = chl.Hydro(nx, ny, nz, ng, chl.RECON_PPMC, chl.PREC_MIXED, **kw)
+        assert kw or (hy.config().tile1 == 2) == wide
+        hy.run(D, *w, G, 0.0, 1e30, 2)
+        out.append(D.download())
+    assert np.array_equal(out[0], out[1])
