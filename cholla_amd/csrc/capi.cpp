@@ -197,15 +197,12 @@ int EnqueueStep(chl_hydro *h, double *U, double dx, double dy, double dz, double
     CHL_HIP(chl::LaunchDtAdvance(h->dti(), h->dt(), h->t(), *tout, kCfl, h->nstep(), h->stream));
   if (h->one_d) {
     const int n = c.nx;
-    // the dt reduction rides on the last kernel of the step: the one-block stage 2, or with
-    // dual energy the energy sync (any number of blocks)
+    // the dt reduction rides on the last kernel of the step: stage 2, or with dual energy the
+    // energy sync
     // (stage 1 zeroes the accumulator in-kernel, so a captured step holds no memset node)
-    bool fuse_dt = update_grid && (n <= 1024 || c.dual_energy);
     CHL_HIP(chl::LaunchVl1d(U, reinterpret_cast<double *>(h->W), n, ng, c.reconstruction, SolverKind(c.riemann),
-                            c.dual_energy != 0, c.precision, dx, dt_dev, dt_host, gamma, fuse_dt ? h->dti() : nullptr,
-                            update_grid ? h->dti() : nullptr, h->grav, h->stream));
-    if (update_grid && !fuse_dt)
-      CHL_HIP(chl::LaunchCalcDt(U, n, 1, 1, ng, dx, dy, dz, gamma, h->dti(), h->num_cu, h->stream));
+                            c.dual_energy != 0, c.precision, dx, dt_dev, dt_host, gamma,
+                            update_grid ? h->dti() : nullptr, update_grid ? h->dti() : nullptr, h->grav, h->stream));
     if (fill) CHL_HIP(chl::LaunchGhostFill(U, c.nx, c.ny, c.nz, c.n_fields, ng, c.bc_flags, h->stream));
     return CHL_OK;
   }

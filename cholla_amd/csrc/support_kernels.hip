@@ -380,8 +380,9 @@ __global__ void TurbulenceIcKernel(double *U, int n, int ng, int n_modes, const 
 // Update_Conserved_Variables_1D_half (hydro_cuda.cu:222-263): the pressure from the
 // total energy, the neighbours' velocities by division.
 template <class P, bool DE>
-__global__ void Vl1dStage1Kernel(const double *U, double *W, int n, double dx, const double *dt_dev, double dt_host,
-                                 double gamma, unsigned long long *dti_reset)
+__global__ void __launch_bounds__(256) Vl1dStage1Kernel(const double *U, double *W, int n, double dx,
+                                                        const double *dt_dev, double dt_host, double gamma,
+                                                        unsigned long long *dti_reset)
 {
   using T = typename P::T;
   int id  = blockIdx.x * blockDim.x + threadIdx.x;
@@ -418,9 +419,16 @@ __global__ void Vl1dStage1Kernel(const double *U, double *W, int n, double dx, c
 // on top of the full-step pdV source Vl1dPdvKernel added; PCM with DE passes the half state
 // through with its conserved GasEnergy (PCM_Reconstruction_1D, pcm_cuda.cu:13-97), so its
 // faces are stage 1's PCM faces on W.
+//
+// A line is a handful of workgroups, so a thread's own chain bounds the launch: three
+// reconstructions and two solves.  Workgroups of 256, one wave per SIMD, leave it the registers
+// (up to 254); compiled for the one workgroup of 1024 that an earlier dt reduction needed it
+// had 128 and spilled, more so with the shared reciprocals of hydro_physics.hpp.  (1000 cells,
+// Roe, PLMC, FP64: a step in 24.2 us, with 1024 threads 44.8, with compiled quotients there 40.4.)
 template <class P, int RK, bool DE>
-__global__ void Vl1dStage2Kernel(double *U, const double *W, int n, int ng, double dx, const double *dt_dev,
-                                 double dt_host, double gamma, unsigned long long *dti, GravSpec grav)
+__global__ void __launch_bounds__(256) Vl1dStage2Kernel(double *U, const double *W, int n, int ng, double dx,
+                                                        const double *dt_dev, double dt_host, double gamma,
+                                                        unsigned long long *dti, GravSpec grav)
 {
   using T         = typename P::T;
   int id          = blockIdx.x * blockDim.x + threadIdx.x;
@@ -532,8 +540,8 @@ __global__ void Vl1dSyncKernel(double *U, int n, int ng, double dx, double gamma
 // the PCM build): the x face i+1/2 and y face j+1/2 of every cell with a neighbour there,
 // from the conserved states as they are.  Thread 0 clears the step's dt reduction.
 template <class P, bool DE = false>
-__global__ void Vl2dPcmFluxKernel(const double *U, double *Fx, double *Fy, int nx, int ny, double gamma,
-                                  unsigned long long *dti_reset)
+__global__ void __launch_bounds__(256) Vl2dPcmFluxKernel(const double *U, double *Fx, double *Fy, int nx, int ny,
+                                                         double gamma, unsigned long long *dti_reset)
 {
   using T       = typename P::T;
   const long nc = long(nx) * ny;
@@ -766,7 +774,8 @@ __device__ __forceinline__ void DirSlots(int dir, int &o1, int &o2, int &o3)
 // interface layout (plmc_cuda.cu:24-300, ppmc_cuda.cu:540-695): Q_L at cell i,
 // Q_R at cell i-1 along dir, conserved variables in global momentum slots.
 template <int RK, bool DE = false>
-__global__ void ReconGridKernel(const double *U, double *QL, double *QR, int nx, int ny, int nz, double gamma, int dir)
+__global__ void __launch_bounds__(64) ReconGridKernel(const double *U, double *QL, double *QR, int nx, int ny, int nz,
+                                                      double gamma, int dir)
 {
   constexpr int r  = ReconTraits<RK>::kRadius;
   constexpr int NS = 2 * r + 1;
@@ -846,8 +855,8 @@ __global__ void ReconGridKernel(const double *U, double *QL, double *QR, int nx,
 // HllPolicy / RoePolicy / ExactPolicy, Calculate_HLL_Fluxes_CUDA (hll_cuda.cu:19-268) /
 // Calculate_Roe_Fluxes_CUDA (roe_cuda.cu:19-400) / Calculate_Exact_Fluxes_CUDA (exact_cuda.cu:20-334)
 template <class P, bool DE = false>
-__global__ void RiemannGridKernel(const double *QL, const double *QR, double *F, int nx, int ny, int nz, double gamma,
-                                  int dir)
+__global__ void __launch_bounds__(64) RiemannGridKernel(const double *QL, const double *QR, double *F, int nx, int ny,
+                                                        int nz, double gamma, int dir)
 {
   const size_t nc = size_t(nx) * ny * nz;
   size_t t        = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1014,23 +1023,20 @@ static hipError_t LaunchVl1dP(double *U, double *W, int n, int ng, int recon, do
     hipLaunchKernelGGL(Vl1dSyncKernel, dim3(nb), dim3(256), 0, s, U, n, ng, dx, gamma, dti);
     return hipGetLastError();
   } else {
-    // one block when a dt reduction is fused so the block max is the grid max
-    const unsigned nb2 = dti ? 1u : nb;
-    const int tpb      = dti ? 1024 : 256;
     if (recon == kPPMC) {
-      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPPMC, false>), dim3(nb2), dim3(tpb), 0, s, U, W, n, ng, dx, dt_dev, dt,
+      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPPMC, false>), dim3(nb), dim3(256), 0, s, U, W, n, ng, dx, dt_dev, dt,
                          gamma, dti, grav);
     } else if (recon == kPLMC) {
-      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPLMC, false>), dim3(nb2), dim3(tpb), 0, s, U, W, n, ng, dx, dt_dev, dt,
+      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPLMC, false>), dim3(nb), dim3(256), 0, s, U, W, n, ng, dx, dt_dev, dt,
                          gamma, dti, grav);
     } else if (recon == kPLMP) {
-      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPLMP, false>), dim3(nb2), dim3(tpb), 0, s, U, W, n, ng, dx, dt_dev, dt,
+      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPLMP, false>), dim3(nb), dim3(256), 0, s, U, W, n, ng, dx, dt_dev, dt,
                          gamma, dti, grav);
     } else if (recon == kPPMP) {
-      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPPMP, false>), dim3(nb2), dim3(tpb), 0, s, U, W, n, ng, dx, dt_dev, dt,
+      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPPMP, false>), dim3(nb), dim3(256), 0, s, U, W, n, ng, dx, dt_dev, dt,
                          gamma, dti, grav);
     } else if (recon == kPCM) {
-      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPCM, false>), dim3(nb2), dim3(tpb), 0, s, U, W, n, ng, dx, dt_dev, dt,
+      hipLaunchKernelGGL((Vl1dStage2Kernel<P, kPCM, false>), dim3(nb), dim3(256), 0, s, U, W, n, ng, dx, dt_dev, dt,
                          gamma, dti, grav);
     } else {
       return hipErrorInvalidValue;
@@ -1056,7 +1062,6 @@ hipError_t LaunchVl1d(double *U, double *W, int n, int ng, int recon, int rieman
                       const double *dt_dev, double dt, double gamma, unsigned long long *dti,
                       unsigned long long *dti_reset, const GravSpec &grav, hipStream_t s)
 {
-  if (dti && n > 1024 && !de) return hipErrorInvalidValue;
   if (recon != kPPMC && recon != kPLMC && recon != kPLMP && recon != kPPMP && recon != kPCM) return hipErrorInvalidValue;
   switch (form) {
     case PolicyExact::kId:

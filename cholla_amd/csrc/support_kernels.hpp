@@ -36,7 +36,7 @@ hipError_t LaunchDtAdvance(unsigned long long *dti, double *dt_dev, double *t_de
                            int *n_step, hipStream_t s, bool take = false);
 hipError_t LaunchTurbulenceIc(double *U, int n, int ng, int n_modes, const double *modes, double vscale, double rho,
                               double p, double gamma, hipStream_t s);
-// dti: reduce the next inverse dt into it (stage 2 with one block, or the DE energy sync);
+// dti: reduce the next inverse dt into it (stage 2, or the DE energy sync);
 // dti_reset: zero it first, from stage 1 (both may be the same pointer).
 // form: the arithmetic form's id (PolicyExact::kId, PolicyFast::kId, PolicyMixed::kId)
 hipError_t LaunchVl1d(double *U, double *W, int n, int ng, int recon, int riemann, bool de, int form, double dx,

@@ -310,9 +310,9 @@ def test_linear_wave_system(recon):
 
 @pytest.mark.parametrize("use_graph", [False, True])
 def test_sod_1d_large_unfused_dt(use_graph):
-    """A 1D tube above 1024 cells without dual energy: the next inverse dt is its own grid-wide
-    reduction after the step, whose accumulator stage 1 zeroes in-kernel (no memset in the
-    captured step).  2000 cells, PPMC + HLLC, to t = 0.05: bit-identical to the oracle."""
+    """A 1D tube above 1024 cells without dual energy: stage 2's workgroups reduce the next
+    inverse dt into an accumulator that stage 1 zeroes in-kernel (no memset in the captured
+    step).  2000 cells, PPMC + HLLC, to t = 0.05: bit-identical to the oracle."""
     U, nx, dx = sod_ic(n_real=2000, ng=4)
     ng = 4
     orc.set_boundaries(U, nx, 1, 1, 5, ng, [3, 3, 0, 0, 0, 0])
