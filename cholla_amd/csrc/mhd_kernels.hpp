@@ -348,6 +348,67 @@ __device__ __forceinline__ void PlmcCellM(const double *U, int x, int y, int z, 
                 LoadDataM<P>(U, x + di, y + dj, z + dk, nx, ny, n, dir, g), g, Lp, Rm);
 }
 
+// reconstruction::PPM_Single_Variable, src/reconstruction/reconstruction.h:794-901, FP64: the
+// values PpmSingle forms (bit for bit under PolicyExact), by the reference's own expressions.
+// Seven characteristics are limited here where hydro has five, and what bounds the launch is the
+// waves that fit: the shared terms of PpmSingle keep more values live, 230 VGPRs for an x-face
+// tile of the exact form and 66 spills in the 168 the fast one is held to, against 162 and 164
+// with these.  Orszag-Tang 256^3, PPMC, a step: exact 12.47 ms (PpmSingle 12.71), FP64 11.60
+// (12.70).
+template <class P>
+__device__ __forceinline__ void PpmSingleM(typename P::T im2, typename P::T im1, typename P::T i0, typename P::T ip1,
+                                           typename P::T ip2, typename P::T &L_iph, typename P::T &R_imh)
+{
+  using T = typename P::T;
+  static_assert(sizeof(T) == 8, "the FP32 form is PpmSingleReduced");
+  const T C2   = T(1.25);
+  const T inv6 = T(1.0 / 6.0);
+  auto neg         = [](T x) { return x < T(0); };
+  auto limit_iface = [&](T c_i, T c_im1, T iface, T s2_i, T s2_im1) -> T {
+    const T s2c     = T(3.0) * (c_im1 + c_i - T(2.0) * iface);
+    const bool same = (neg(s2c) == neg(s2_im1)) && (neg(s2c) == neg(s2_i));
+    const T mag     = Fmin(C2 * Fabs(s2_im1), Fmin(C2 * Fabs(s2_i), Fabs(s2c)));
+    const T limited = same ? (neg(s2c) ? -mag : mag) : T(0.0);
+    const T extr    = T(0.5) * (c_im1 + c_i) - Div<P>(limited, T(6.0), inv6);
+    return ((iface - c_im1) * (c_i - iface) < T(0.0)) ? extr : iface;
+  };
+  const T sL = i0 - im1, sR = ip1 - i0;
+  const T avg_im1 = T(0.5) * sL + T(0.5) * (im1 - im2);
+  const T avg_i   = T(0.5) * sR + T(0.5) * sL;
+  const T avg_ip1 = T(0.5) * (ip2 - ip1) + T(0.5) * sR;
+  T R = T(0.5) * (im1 + i0) + Div<P>(avg_im1 - avg_i, T(6.0), inv6);
+  T L = T(0.5) * (i0 + ip1) + Div<P>(avg_i - avg_ip1, T(6.0), inv6);
+
+  const T s2_im1 = im2 + i0 - T(2.0) * im1;
+  const T s2_i   = im1 + ip1 - T(2.0) * i0;
+  const T s2_ip1 = i0 + ip2 - T(2.0) * ip1;
+  R = limit_iface(i0, im1, R, s2_i, s2_im1);
+  L = limit_iface(ip1, i0, L, s2_ip1, s2_i);
+
+  const T s2_face   = T(6.0) * (R + L - T(2.0) * i0);
+  const bool smooth = neg(s2_im1) == neg(s2_i) && neg(s2_im1) == neg(s2_ip1) && neg(s2_im1) == neg(s2_face);
+  const T mag       = Fmin(Fmin(C2 * Fabs(s2_im1), C2 * Fabs(s2_i)), Fmin(C2 * Fabs(s2_ip1), Fabs(s2_face)));
+  const T limited   = smooth ? (neg(s2_face) ? -mag : mag) : T(0.0);
+  const T cell_max  = Fmax(Fmax(Fmax(Fmax(Fabs(im2), Fabs(im1)), Fabs(i0)), Fabs(ip1)), Fabs(ip2));
+  T ratio;
+  if constexpr (P::kExact) {
+    ratio = limited / s2_face;
+  } else {
+    ratio = QuotOnce(limited, s2_face);
+  }
+  const T rho = (Fabs(s2_face) > T(1.0e-12) * cell_max) ? ratio : T(0.0);
+
+  const T sfl = i0 - R, sfr = L - i0;
+  const bool extremum = (sfl * sfr) <= T(0.0) || (sR * sL) <= T(0.0);
+  const bool flatten  = rho <= (T(1.0) - T(1.0e-12));
+  const T R_ext  = flatten ? i0 - rho * sfl : R;
+  const T L_ext  = flatten ? i0 + rho * sfr : L;
+  const T R_mono = (Fabs(sfl) >= T(2.0) * Fabs(sfr)) ? i0 - T(2.0) * sfr : R;
+  const T L_mono = (Fabs(sfr) >= T(2.0) * Fabs(sfl)) ? i0 + T(2.0) * sfl : L;
+  R_imh = extremum ? R_ext : R_mono;
+  L_iph = extremum ? L_ext : L_mono;
+}
+
 // PPMC_VL with MHD for one cell (ppmc_cuda.cu:540-695) from the primitives of the cell (c0)
 // and its neighbours along dir (cm2, cm1, cp1, cp2): the 5-cell stencil projected on the
 // cell's seven MHD characteristics, PPM_Single_Variable on each (the reduced FP32 form under
@@ -376,7 +437,7 @@ __device__ __forceinline__ void PpmcPrimsM(const PrimM<typename P::T> &cm2, cons
     if constexpr (P::kId == PolicyMixed::kId) {
       PpmSingleReduced(im2, im1, i0, ip1, ip2, l, r);
     } else {
-      PpmSingle<P>(im2, im1, i0, ip1, ip2, l, r);
+      PpmSingleM<P>(im2, im1, i0, ip1, ip2, l, r);
     }
   };
   ppm(am2.a0, am1.a0, a0.a0, ap1.a0, ap2.a0, L.a0, R.a0);

@@ -75,3 +75,10 @@ def test_line_kernels_do_not_spill(kernels, prefix):
     every solver and reconstruction."""
     spills = {n: k["vgpr_spill_count"] for n, k in matching(kernels, prefix).items() if k["vgpr_spill_count"]}
     assert not spills
+
+
+@pytest.mark.parametrize("form", ["PolicyExact", "PolicyFast"])
+def test_mhd_ppmc_x_faces_hold_three_waves(kernels, form):
+    """The FP64 x-face launch of the MHD step with PPMC: three waves per SIMD, nothing spilled."""
+    k = matching(kernels, f"mhd::MhdFlux2TileKernel<{form}, 2>").popitem()[1]
+    assert k["vgpr_spill_count"] == 0 and k["vgpr_count"] <= 168
