@@ -972,9 +972,13 @@ __device__ __forceinline__ double MhdInverseCrossingTimeOf(double d, double mx, 
   const double dinv = QuotOnce(1.0, d);
   const double vx = mx * dinv, vy = my * dinv, vz = mz * dinv;
   const double gasP = PressurePrimM(E, d, vx, vy, vz, g, bx, by, bz);
-  const double cf   = Magnetosonic<PolicyExact>(d, gasP, bx, by, bz, g, 1.0);
-  // (compiled divisions: hoisted reciprocals of dx, dy, dz put MhdFlux1MarchKernel into spills,
-  // 0.96 -> 1.03 ms on Orszag-Tang 256^3)
+  // The fast speed of Magnetosonic<PolicyExact> (the same bits).  This is folded into the loads
+  // of MhdFlux1MarchKernel, which has 128 VGPRs and none to spare: SqrtUnscaled in place of the
+  // compiled roots spilled two (Orszag-Tang 256^3: 964 us now, 994 with them), hoisted
+  // reciprocals of dx, dy and dz in place of the divisions more (1030 us).
+  const double bx2 = bx * bx, b2 = bx2 + ((by * by) + (bz * bz)), t1 = g * gasP + b2;
+  const double t2  = __builtin_sqrt((t1 * t1) - 4. * g * gasP * bx2);
+  const double cf  = __builtin_sqrt(QuotOnce(t1 + t2, 2.0 * Fmax(d, kTinyNumber)));
   double m          = Fmax((Fabs(vx) + cf) / dx, (Fabs(vy) + cf) / dy);
   m                 = Fmax(m, (Fabs(vz) + cf) / dz);
   return Fmax(m, 0.0);

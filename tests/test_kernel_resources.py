@@ -82,3 +82,10 @@ def test_mhd_ppmc_x_faces_hold_three_waves(kernels, form):
     """The FP64 x-face launch of the MHD step with PPMC: three waves per SIMD, nothing spilled."""
     k = matching(kernels, f"mhd::MhdFlux2TileKernel<{form}, 2>").popitem()[1]
     assert k["vgpr_spill_count"] == 0 and k["vgpr_count"] <= 168
+
+
+def test_mhd_mixed_stage_1_holds_four_waves(kernels):
+    """The mixed stage-1 march of the MHD step is compiled for four waves per SIMD, with its dt
+    reduction in registers too."""
+    k = matching(kernels, "mhd::MhdFlux1MarchKernel<PolicyMixed").popitem()[1]
+    assert k["vgpr_spill_count"] == 0 and k["vgpr_count"] <= 128
