@@ -1436,7 +1436,7 @@ __global__ void __launch_bounds__(CTX *CTY) MhdCtUpdateKernel(MhdArgs a, int clo
 {
   using TF         = typename P::T;
   constexpr int NT = CTX * CTY, EX = CTX + 1, EY = CTY + 1;
-  __shared__ CtPlane<TF, CTX + 2, CTY + 2> pl[2];
+  __shared__ CtPlane<TF, CTX + 2, CTY + 2> pl[2];  // (MhdCtChunk counts this LDS)
   __shared__ double eds[3][EY][EX];
   const double dt = FULL ? MhdDt(a) : 0.5 * MhdDt(a);
   if (dt == 0.0) return;

@@ -52,16 +52,32 @@ void MhdFlux2Tiles(const mhd::MhdArgs &a, int lo, int hx, int hy, int hz, hipStr
                      dim3(256), 0, s, a, lo, hx, hy, hz, int(kz));
 }
 
+// The tiles of the CT-update launches, and their planes per workgroup: as many workgroups run on
+// a CU as their LDS admits, three of the mixed form (48 KB of 160) and two of the FP64 ones
+// (72 KB).  Counted as three, these took 12 planes where 16 are faster: Orszag-Tang 128^3 in
+// FP64, the full update 241 us against 206.
+constexpr int kCtX = 32, kCtY = 8;
+template <class P>
+int MhdCtChunk(long columns, int planes)
+{
+  constexpr size_t lds = 2 * sizeof(mhd::CtPlane<typename P::T, kCtX + 2, kCtY + 2>) +
+                         3 * (kCtX + 1) * (kCtY + 1) * sizeof(double);
+  constexpr int per_cu = lds <= 160 * 1024 / 3 ? 3 : 2;
+  static_assert(per_cu * lds <= 160 * 1024, "the workgroups of a CU share its LDS");
+  return MhdChunk(columns, planes, 256 * per_cu, 1.5, 16);
+}
+
 // CT edge fields fused with one stage's update (MhdCtUpdateKernel) over the cells [clo, ch*]
 // and the edges [elo, eh*]: 32 x 8 tiles, z-chunks of up to 16 planes (on Orszag-Tang 256^3
-// these ran 2-5 % faster than 16 x 16 tiles or z-chunks of 8 and 32).
+// these ran 2-5 % faster than 16 x 16 tiles or z-chunks of 8 and 32).  Over boxes of 32^3 to
+// 256^3 the chunk taken costs a step 0.05 % in the mean against the best of all, 1.1 % at worst.
 template <class P, bool FULL>
 void MhdCtUpdate(const mhd::MhdArgs &a, int clo, int chx, int chy, int chz, int elo, int ehx, int ehy, int ehz,
                  hipStream_t s)
 {
-  constexpr int CTX = 32, CTY = 8;
+  constexpr int CTX = kCtX, CTY = kCtY;
   const int columns    = ((chx - clo + CTX) / CTX) * ((chy - clo + CTY) / CTY);
-  const int kchunk     = MhdChunk(columns, chz - clo + 1, 768, 1.5, 16);  // three workgroups per CU
+  const int kchunk     = MhdCtChunk<P>(columns, chz - clo + 1);
   const unsigned tiles = unsigned(columns * ((chz - clo + kchunk) / kchunk));
   hipLaunchKernelGGL((mhd::MhdCtUpdateKernel<P, CTX, CTY, FULL>), dim3((tiles + 7) / 8 * 8), dim3(CTX * CTY), 0, s, a,
                      clo, chx, chy, chz, elo, ehx, ehy, ehz, kchunk);

@@ -13,6 +13,7 @@ import subprocess
 import pytest
 
 import cholla_amd as chl
+from cholla_amd import build
 
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 READELF = shutil.which("llvm-readelf") or "/opt/rocm/llvm/bin/llvm-readelf"
@@ -36,10 +37,10 @@ def code_objects(blob):
 
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
-    """Demangled kernel name (without its arguments) -> VGPRs and spilled VGPRs."""
+    """Demangled kernel name (without its arguments) -> VGPRs, spilled VGPRs and LDS."""
     if not os.path.exists(chl.LIB_PATH) or not os.path.exists(READELF):
         pytest.skip("needs the built library and llvm-readelf")
-    names, found = [], []
+    entries = []  # one per kernel; .agpr_count is the first key of each
     with open(chl.LIB_PATH, "rb") as f:
         blob = f.read()
     d = tmp_path_factory.mktemp("co")
@@ -48,18 +49,18 @@ def kernels(tmp_path_factory):
         path.write_bytes(co)
         notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
         path.unlink()
-        entry = None
         for line in notes.splitlines():
             key, _, value = line.strip().lstrip("- ").partition(":")
-            if key == ".name" and value.strip().startswith("_Z"):
-                names.append(value.strip())
-                entry = {}
-                found.append(entry)
-            elif entry is not None and key in (".vgpr_count", ".vgpr_spill_count"):
-                entry[key[1:]] = int(value)
+            if key == ".agpr_count":
+                entries.append({})
+            if key in (".vgpr_count", ".vgpr_spill_count", ".group_segment_fixed_size"):
+                entries[-1][key[1:]] = int(value)
+            elif key == ".name" and value.strip().startswith("_Z"):
+                entries[-1]["name"] = value.strip()
+    names = [e.pop("name") for e in entries]
     out = subprocess.run(["c++filt"], input="\n".join(names), capture_output=True, text=True, check=True).stdout
     short = (n.replace("void ", "").replace("chl::", "").split("(")[0] for n in out.splitlines())
-    return dict(zip(short, found))
+    return dict(zip(short, entries))
 
 
 def matching(kernels, prefix):
@@ -89,3 +90,22 @@ def test_mhd_mixed_stage_1_holds_four_waves(kernels):
     reduction in registers too."""
     k = matching(kernels, "mhd::MhdFlux1MarchKernel<PolicyMixed").popitem()[1]
     assert k["vgpr_spill_count"] == 0 and k["vgpr_count"] <= 128
+
+
+def test_mhd_ct_chunks_count_the_workgroups_a_cu_holds(kernels, tmp_path):
+    """The planes per workgroup of the CT updates on a 128^3 box (64 columns of tiles): one round
+    of the workgroups that the kernel's LDS admits, 8 chunks of 16 for the FP64 forms' two per CU
+    and 11 of 12 for the mixed form's three."""
+    per_cu = {}
+    for form in ("PolicyExact", "PolicyFast", "PolicyMixed"):
+        lds = {k["group_segment_fixed_size"] for k in matching(kernels, f"mhd::MhdCtUpdateKernel<{form}").values()}
+        per_cu[form] = 160 * 1024 // max(lds)
+    assert per_cu == {"PolicyExact": 2, "PolicyFast": 2, "PolicyMixed": 3}
+    src = tmp_path / "chunk.hip"
+    src.write_text('#include "mhd_launch.hpp"\n#include <cstdio>\n'
+                   "int main() { std::printf(\"%d %d %d\", chl::MhdCtChunk<chl::PolicyExact>(64, 128),"
+                   " chl::MhdCtChunk<chl::PolicyFast>(64, 128), chl::MhdCtChunk<chl::PolicyMixed>(64, 128)); }\n")
+    exe = tmp_path / "chunk"
+    subprocess.run([build.hipcc(), *build.COMMON, "-O0", "--cuda-host-only", f"-I{build.CSRC}", str(src), "-o", str(exe)],
+                   check=True, capture_output=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout == "16 16 12"
