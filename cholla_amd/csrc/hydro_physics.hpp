@@ -124,9 +124,15 @@ struct Char5 {
 // 307 divisions made 40 % of the reference-order stage 2.  A quotient here is 4 instructions
 // and a reciprocal 5; PPMC on KH 256^3, 16x8 tiles: stage 2 5.09 -> 3.99 ms, stage 1 1.55 ->
 // 1.31 ms (reference order).  The result has the compiled division's bits wherever that does
-// not scale, which is for |n| >= 2^-969 or n = 0, |n / d| < 2^768, and d, 1/d and n/d normal;
-// outside, a tiny quotient may be an ulp off.  Zeros, infinities and NaN come out as IEEE
-// division's (v_div_fixup).
+// not scale, which is for |n| >= 2^-969 or n = 0, |n / d| < 2^768, and d, 1/d and n/d normal.
+// Zeros, infinities and NaN come out as IEEE division's (v_div_fixup).  Outside, a quotient of
+// a tiny n may be an ulp off, and one by a subnormal d is NaN.  Denominators here are densities,
+// pressures, sound speeds and differences of signal speeds (floors of 1e-20 or sums with such)
+// or cell widths, but for the slopes and limiters, whose values may be the far tail of a
+// velocity: the limiters keep subnormal denominators out (PpmSingle), the sum of two slopes is
+// not subnormal where their product is positive, and the reference-order form, which owes the
+// reference's bits there too, divides in full where a numerator is a product of two such values
+// or the denominator is one (SlopeQuot, PpmSingle).
 __device__ __forceinline__ double RcpRefined(double d)
 {
   double r = __builtin_amdgcn_rcp(d);
@@ -356,6 +362,19 @@ __device__ __forceinline__ Prim<typename P::T> CharToPrim(const Prim<typename P:
 }
 
 // ---------------------------------------------------------------------------- PPM limiter
+// The limiters' round-off bound on a second difference (the reference's 1e-12 of the values).
+// The non-exact forms, whose quotient by a subnormal difference would be NaN, add the least
+// normal number (in the product's FMA) and so take those as round-off too.
+template <class P>
+__device__ __forceinline__ double RoundOff(double cell_max)
+{
+  if constexpr (P::kExact) {
+    return 1.0e-12 * cell_max;
+  } else {
+    return 1.0e-12 * cell_max + 2.2250738585072014e-308;
+  }
+}
+
 // Whether all of the arguments' sign tests agree, as lane masks (no branches).
 __device__ __forceinline__ bool Agree(bool a, bool b, bool c) { return !((a ^ b) | (a ^ c)); }
 __device__ __forceinline__ bool Agree(bool a, bool b, bool c, bool d) { return !((a ^ b) | (a ^ c) | (a ^ d)); }
@@ -411,15 +430,15 @@ __device__ __forceinline__ void PpmSingle(typename P::T im2, typename P::T im1, 
   cell_max   = Fmax(cell_max, Fabs(ip1));
   cell_max   = Fmax(cell_max, Fabs(ip2));
 
-  // The 1e-12 round-off guard is the reference's.  (The exact form divides in full:
-  // s2_face may be subnormal.)
+  // s2_face may be subnormal, in the far tail of a velocity: the exact form divides in full, the
+  // others take it as round-off.
   T ratio;
   if constexpr (P::kExact) {
     ratio = mag / Fabs(s2_face);
   } else {
     ratio = QuotOnce(mag, Fabs(s2_face));
   }
-  const T rho = (smooth & (Fabs(s2_face) > T(1.0e-12) * cell_max)) ? ratio : T(0.0);
+  const T rho = (smooth & (Fabs(s2_face) > RoundOff<P>(cell_max))) ? ratio : T(0.0);
 
   const T sfl = i0 - R, sfr = L - i0;
   const T sfl2 = T(2.0) * sfl, sfr2 = T(2.0) * sfr;
@@ -554,7 +573,7 @@ __device__ __forceinline__ void PpmSingleCentred(double im2, double im1, double 
   const T mag       = Fmin(Fmin(wl, wp), Fabs(s2face));
   const T cmax      = Fmax(Fmax(Fabs(im2), Fabs(im1)), Fmax(Fabs(ip1), Fabs(ip2))) + Fabs(centre);
   const T ratio     = QuotOnce(mag, Fabs(s2face));
-  const T rho       = (smooth & (Fabs(s2face) > T(1.0e-12) * cmax)) ? ratio : T(0);
+  const T rho       = (smooth & (Fabs(s2face) > RoundOff<PolicyFast>(cmax))) ? ratio : T(0);
   const T R2 = T(-2.0) * R, L2 = T(-2.0) * L;
   const bool extremum = Fmax(R * L, ip1 * im1) >= T(0);  // sfl = -R, sfr = L
   const bool flatten  = extremum & (rho <= (T(1.0) - T(1.0e-12)));
@@ -649,10 +668,23 @@ __device__ __forceinline__ bool ReconPpmc(const Prim<typename P::T> s[5], typena
 }
 
 // ---------------------------------------------------------------------------- PLMC (VL)
-template <typename T>
-__device__ __forceinline__ T VlSlope(T l, T r, T inv_sum)  // Van_Leer_Slope, reconstruction.h:266-272
+// 2 l r / (l + r), the harmonic mean of two slopes of one sign.  The product leaves Quot's range
+// at slopes of 1e-146, which a localised flow's tails hold: the exact form divides in full (its
+// stage 2 is 1-2 % longer for it with PLMC, PLMP and PPMP).
+template <class P>
+__device__ __forceinline__ typename P::T SlopeQuot(typename P::T n, typename P::T d)
 {
-  return (l * r > T(0.0)) ? QuotOnce(T(2.0) * l * r, l + r) : T(0.0);
+  if constexpr (P::kExact) {
+    return n / d;
+  } else {
+    return QuotOnce(n, d);
+  }
+}
+template <class P>
+__device__ __forceinline__ typename P::T VlSlope(typename P::T l, typename P::T r)  // Van_Leer_Slope, reconstruction.h:266-272
+{
+  using T = typename P::T;
+  return (l * r > T(0.0)) ? SlopeQuot<P>(T(2.0) * l * r, l + r) : T(0.0);
 }
 
 // Monotonize lambda, reconstruction.h:519-527
@@ -667,6 +699,19 @@ __device__ __forceinline__ T MonotonizeOne(T left, T right, T centered, T van_le
   return T(0.0);
 }
 
+// The Van Leer slope of PLMP and PPMP (plmp_cuda.cu:340-346): VlSlope, its quotient by Rcp in the
+// non-exact forms.
+template <class P>
+__device__ __forceinline__ typename P::T PlmpHarmonic(typename P::T l, typename P::T r)
+{
+  using T = typename P::T;
+  if constexpr (P::kExact) {
+    return VlSlope<P>(l, r);
+  } else {
+    return l * r > T(0.0) ? Div1<P>(T(2.0) * l * r, l + r) : T(0.0);
+  }
+}
+
 // Interface_Values_PLM, src/reconstruction/plmp_cuda.cu:325-365: the Van Leer limited slope
 // of one primitive variable; lo / hi are the values at the cell's left / right face.
 template <class P>
@@ -675,7 +720,7 @@ __device__ __forceinline__ void PlmpInterface(typename P::T qm, typename P::T q0
 {
   using T = typename P::T;
   const T dL = q0 - qm, dR = qp - q0, dC = T(0.5) * (qp - qm);
-  const T dG = dL * dR > T(0.0) ? Div1<P>(T(2.0) * dL * dR, dL + dR) : T(0.0);
+  const T dG = PlmpHarmonic<P>(dL, dR);
   const T a = Fmin(Fabs(dL), Fabs(dR));
   const T b = Fmin(Fabs(dC), Fabs(dG));
   const T dm = SignOf(dC) * Fmin(T(2.0) * a, b);  // sgn_CUDA, global_cuda.h:41-48
@@ -718,7 +763,7 @@ __device__ __forceinline__ typename P::T LimitedSlope(typename P::T qm, typename
 {
   using T    = typename P::T;
   const T dL = q0 - qm, dR = qp - q0, dC = T(0.5) * (qp - qm);
-  const T dG = dL * dR > T(0.0) ? Div1<P>(T(2.0) * dL * dR, dL + dR) : T(0.0);
+  const T dG = PlmpHarmonic<P>(dL, dR);
   return SignOf(dC) * Fmin(T(2.0) * Fmin(Fabs(dL), Fabs(dR)), Fmin(Fabs(dC), Fabs(dG)));
 }
 
@@ -787,8 +832,8 @@ __device__ __forceinline__ void ReconPlmcCore(const Prim<typename P::T> s[3], co
              T(1.0) * (ip.p - q.p)};
   Prim<T> dC{T(0.5) * (ip.d - im.d), T(0.5) * (ip.vx - im.vx), T(0.5) * (ip.vy - im.vy), T(0.5) * (ip.vz - im.vz),
              T(0.5) * (ip.p - im.p)};
-  Prim<T> dG{VlSlope(dL.d, dR.d, T(0)), VlSlope(dL.vx, dR.vx, T(0)), VlSlope(dL.vy, dR.vy, T(0)),
-             VlSlope(dL.vz, dR.vz, T(0)), VlSlope(dL.p, dR.p, T(0))};
+  Prim<T> dG{VlSlope<P>(dL.d, dR.d), VlSlope<P>(dL.vx, dR.vx), VlSlope<P>(dL.vy, dR.vy),
+             VlSlope<P>(dL.vz, dR.vz), VlSlope<P>(dL.p, dR.p)};
   Char5<T> aL = PrimToChar<P>(qe, dL, cs), aR = PrimToChar<P>(qe, dR, cs), aG = PrimToChar<P>(qe, dG, cs);
   Char5<T> aC;
   if constexpr (P::kExact) {  // the reference projects the centred slope itself
@@ -846,7 +891,7 @@ __device__ __forceinline__ void ReconPlmcScalar(const typename P::T g[3], typena
   T dL     = T(1.0) * (g[1] - g[0]);
   T dR     = T(1.0) * (g[2] - g[1]);
   T dC     = T(0.5) * (g[2] - g[0]);
-  T dG     = VlSlope(dL, dR, T(0));
+  T dG     = VlSlope<P>(dL, dR);
   T dm     = MonotonizeOne(dL, dR, dC, dG);
   const T hp = T(1.0) * T(0.5), hm = T(-1.0) * T(0.5);
   L_iph    = g[1] + hp * dm;

@@ -263,11 +263,6 @@ __device__ __forceinline__ T MonoM(T l, T r, T c, T v)  // Monotonize_Characteri
   return T(0.0);
 }
 template <typename T>
-__device__ __forceinline__ T VlM(T l, T r)  // Van_Leer_Slope
-{
-  return (l * r > T(0.0)) ? QuotOnce(T(2.0) * l * r, l + r) : T(0.0);
-}
-template <typename T>
 __device__ __forceinline__ void LimitM(T &l, T &r, T vm, T v0, T vp)  // Plm_Limit_Interfaces
 {
   r = Fmax(Fmin(v0, vm), r);
@@ -296,8 +291,8 @@ __device__ __forceinline__ void PlmcPrimsM(const PrimM<typename P::T> &cm, const
                     c * (r.p - l.p), T(0),             c * (r.by - l.by), c * (r.bz - l.bz)};
   };
   const PrimM<T> dL = slope(cm, c0, T(1.0)), dR = slope(c0, cp, T(1.0)), dC = slope(cm, cp, T(0.5));
-  const PrimM<T> dG{VlM(dL.d, dR.d), VlM(dL.vx, dR.vx), VlM(dL.vy, dR.vy), VlM(dL.vz, dR.vz),
-                    VlM(dL.p, dR.p), T(0),              VlM(dL.by, dR.by), VlM(dL.bz, dR.bz)};
+  const PrimM<T> dG{VlSlope<P>(dL.d, dR.d), VlSlope<P>(dL.vx, dR.vx), VlSlope<P>(dL.vy, dR.vy), VlSlope<P>(dL.vz, dR.vz),
+                    VlSlope<P>(dL.p, dR.p), T(0),              VlSlope<P>(dL.by, dR.by), VlSlope<P>(dL.bz, dR.bz)};
   const Char7<T> aL = PrimToCharM<P>(c0, dL, e, cs2, inv_d, inv_cs2);
   const Char7<T> aR = PrimToCharM<P>(c0, dR, e, cs2, inv_d, inv_cs2);
   Char7<T> aC;
@@ -352,7 +347,7 @@ __device__ __forceinline__ void PlmcCellM(const double *U, int x, int y, int z, 
 // values PpmSingle forms (bit for bit under PolicyExact), by the reference's own expressions.
 // Seven characteristics are limited here where hydro has five, and what bounds the launch is the
 // waves that fit: the shared terms of PpmSingle keep more values live, 230 VGPRs for an x-face
-// tile of the exact form and 66 spills in the 168 the fast one is held to, against 162 and 164
+// tile of the exact form and 66 spills in the 168 the fast one is held to, against 162 and 166
 // with these.  Orszag-Tang 256^3, PPMC, a step: exact 12.47 ms (PpmSingle 12.71), FP64 11.60
 // (12.70).
 template <class P>
@@ -390,13 +385,8 @@ __device__ __forceinline__ void PpmSingleM(typename P::T im2, typename P::T im1,
   const T mag       = Fmin(Fmin(C2 * Fabs(s2_im1), C2 * Fabs(s2_i)), Fmin(C2 * Fabs(s2_ip1), Fabs(s2_face)));
   const T limited   = smooth ? (neg(s2_face) ? -mag : mag) : T(0.0);
   const T cell_max  = Fmax(Fmax(Fmax(Fmax(Fabs(im2), Fabs(im1)), Fabs(i0)), Fabs(ip1)), Fabs(ip2));
-  T ratio;
-  if constexpr (P::kExact) {
-    ratio = limited / s2_face;
-  } else {
-    ratio = QuotOnce(limited, s2_face);
-  }
-  const T rho = (Fabs(s2_face) > T(1.0e-12) * cell_max) ? ratio : T(0.0);
+  const T ratio     = SlopeQuot<P>(limited, s2_face);
+  const T rho       = (Fabs(s2_face) > RoundOff<P>(cell_max)) ? ratio : T(0.0);
 
   const T sfl = i0 - R, sfr = L - i0;
   const bool extremum = (sfl * sfr) <= T(0.0) || (sR * sL) <= T(0.0);

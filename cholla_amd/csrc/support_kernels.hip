@@ -495,7 +495,7 @@ __global__ void Vl1dPdvKernel(double *U, int n, int ng, double dx, const double 
   const double vx = U[n + id] * d_inv, vy = U[2 * n + id] * d_inv, vz = U[3 * n + id] * d_inv;
   const double E = U[4 * n + id], GE = U[5 * n + id];
   const double E_kin  = 0.5 * d * (vx * vx + vy * vy + vz * vz);
-  const double pr     = Fmax(PressureFromDE(E, E - E_kin, GE, gamma), kTinyNumber);
+  const double pr     = LinePressureFromDE(E, E - E_kin, GE, gamma);
   const double vx_imo = U[n + id - 1] / U[id - 1], vx_ipo = U[n + id + 1] / U[id + 1];
   U[5 * n + id] += 0.5 * pr * (dtodx * (vx_imo - vx_ipo));
 }
@@ -635,7 +635,7 @@ __global__ void Vl2dPdvKernel(double *U, int nx, int ny, int ng, double dx, doub
   const double d = U[id], d_inv = 1.0 / d;
   const double vx = U[nc + id] * d_inv, vy = U[2 * nc + id] * d_inv, vz = U[3 * nc + id] * d_inv;
   const double E = U[4 * nc + id], GE = U[5 * nc + id];
-  const double pr = Fmax(PressureFromDE(E, E - 0.5 * d * (vx * vx + vy * vy + vz * vz), GE, gamma), kTinyNumber);
+  const double pr = LinePressureFromDE(E, E - 0.5 * d * (vx * vx + vy * vy + vz * vz), GE, gamma);
   const long imo = id - 1, ipo = id + 1, jmo = id - nx, jpo = id + nx;
   const double vx_imo = U[nc + imo] / U[imo], vx_ipo = U[nc + ipo] / U[ipo];
   const double vy_jmo = U[2 * nc + jmo] / U[jmo], vy_jpo = U[2 * nc + jpo] / U[jpo];
