@@ -521,7 +521,8 @@ int chl_hydro_create(const chl_hydro_config *cfg, chl_hydro **out)
   chl_hydro_config c = *cfg;
   CHL_TRY(chl_capi::PrepareConfig(c));
   auto *h    = new chl_hydro();
-  h->tile2_auto = cfg->tile2 < 0;
+  h->tile2_auto   = cfg->tile2 < 0;
+  h->kchunk2_auto = cfg->kchunk2 <= 0;
   h->one_d   = c.ny == 1 && c.nz == 1;
   h->two_d   = c.nz == 1 && c.ny > 1;
   h->n_cells = size_t(c.nx) * c.ny * c.nz;
@@ -733,12 +734,16 @@ int chl_hydro_set_static_gravity(chl_hydro *h, int custom_grav, int x_off, int y
   const bool grav3d = custom_grav != 0 && !h->one_d && !h->two_d;
   if (grav3d && c.tile2 >= chl::kNumDeTiles) {
     if (!h->tile2_auto) return Fail(CHL_ERR_UNSUPPORTED, "3D static gravity is built for stage-2 tile shapes 0 and 1");
-    // the library's default stage-2 tile has no gravity kernel: take the 16x16 one
-    h->cfg.tile2 = 1;
-    if (h->graph) {
-      (void)hipGraphExecDestroy(h->graph);
-      h->graph = nullptr;
-    }
+    // the stage-2 tile picked for this box has no gravity kernel: tile and z-chunk are picked
+    // again among those that have one, and put back when gravity is taken off
+    h->no_grav_tile2 = c.tile2, h->no_grav_kchunk2 = c.kchunk2;
+    int tile = -1, kchunk = h->kchunk2_auto ? 0 : c.kchunk2;
+    const std::vector<chl_capi::StageExtent> box{{c.nx - 2 * c.n_ghost, c.ny - 2 * c.n_ghost, c.nz - 2 * c.n_ghost}};
+    chl_capi::PickLaunchShape(2, c.precision, c.reconstruction, c.dual_energy != 0, true, box, tile, kchunk);
+    h->cfg.tile2 = tile, h->cfg.kchunk2 = kchunk;
+  } else if (custom_grav == 0 && h->no_grav_tile2 >= 0) {
+    h->cfg.tile2 = h->no_grav_tile2, h->cfg.kchunk2 = h->no_grav_kchunk2;
+    h->no_grav_tile2 = -1;
   }
   chl::GravSpec g{custom_grav, {x_off, y_off, z_off}, {xbound, ybound, zbound}};
   const chl::GravSpec &o = h->grav;
@@ -825,6 +830,7 @@ int chl_hydro_autotune(chl_hydro *h, const double *U, double dx, double dy, doub
   (void)hipFree(S);
   if (rc != CHL_OK) return rc;
   c.tile1 = b_t1, c.tile2 = b_t2, c.kchunk1 = b_k1, c.kchunk2 = b_k2;
+  h->no_grav_tile2 = -1;
   if (h->graph) {
     (void)hipGraphExecDestroy(h->graph);
     h->graph = nullptr;

@@ -28,9 +28,12 @@ struct chl_hydro {
   chl_hydro_config cfg{};
   size_t n_cells = 0;
   bool one_d     = false;
-  bool two_d     = false;  // nz == 1 < ny: the unfused 2D step, W holds its scratch
+  bool two_d     = false;  // nz == 1 < ny: W holds the fused 2D step's half state or the unfused one's scratch
   chl::GravSpec grav{};    // static gravity (chl_hydro_set_static_gravity); id 0 = none
-  bool tile2_auto = false; // the caller left tile2 to the library (-1)
+  bool tile2_auto   = false;  // the caller left tile2 to the library (-1)
+  bool kchunk2_auto = false;  // and kchunk2 (<= 0)
+  // stage 2's launch shape before static gravity took its tile from it (tile -1: it did not)
+  int no_grav_tile2 = -1, no_grav_kchunk2 = 0;
   int num_cu     = 256;
   void *W        = nullptr;  // half-step primitives (+ the pdV sources with dual energy)
   size_t W_bytes = 0;

@@ -233,3 +233,25 @@ def test_static_gravity_limits():
     hy.set_static_gravity(1)
     assert hy.config().tile2 == 1
     hy.close()
+
+
+def test_static_gravity_takes_the_shape_picked_for_its_tiles():
+    """A stage-2 tile and z-chunk left to the library are picked together again for gravity: those
+    of a handle made with the 16x16 tile (196 x 100 x 16 real cells: one plane, where the 32x16
+    tile's chunk is 4).  An explicit chunk stays, and without gravity the first shape is back."""
+    ng, dims = 3, (202, 106, 22)
+    shape = lambda h: (h.config().tile2, h.config().kchunk2)  # noqa: E731
+    hy = chl.Hydro(*dims, ng, chl.RECON_PLMC, chl.PREC_FP64)
+    narrow = chl.Hydro(*dims, ng, chl.RECON_PLMC, chl.PREC_FP64, tile2=1)
+    first = shape(hy)
+    assert first[0] >= 2 and first[1] != shape(narrow)[1]
+    hy.set_static_gravity(1)
+    assert shape(hy) == shape(narrow)
+    hy.set_static_gravity(0)
+    assert shape(hy) == first
+    given = chl.Hydro(*dims, ng, chl.RECON_PLMC, chl.PREC_FP64, kchunk2=7)
+    tile = given.config().tile2
+    given.set_static_gravity(1)
+    assert shape(given) == (1, 7)
+    given.set_static_gravity(0)
+    assert shape(given) == (tile, 7)
