@@ -8,6 +8,7 @@
 #include <limits>
 #include <random>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/cholla_amd.h"
@@ -787,42 +788,42 @@ int chl_hydro_autotune(chl_hydro *h, const double *U, double dx, double dy, doub
   const bool narrow = c.dual_energy || c.riemann != CHL_RIEMANN_HLLC || c.reconstruction == CHL_RECON_PCM ||
                      c.reconstruction == CHL_RECON_PLMP || c.reconstruction == CHL_RECON_PPMP || h->grav.id != 0;
   const int ntiles  = narrow ? chl::kNumDeTiles : chl::kNumTiles;
-  std::vector<int> chunks = {8, 16, 32, 64, 128};
+  // the shape in hand (the rule's z-chunks may be shorter), then every tile with chunks of 8 to
+  // 128 planes
+  auto shapes = [&](int tile, int kchunk, int planes) {
+    std::vector<std::pair<int, int>> v{{tile, kchunk}};
+    for (int t = 0; t < ntiles; t++)
+      for (int kc : {8, 16, 32, 64, 128})
+        if (kc == 8 || kc <= 2 * planes) v.push_back({t, std::min(kc, planes)});
+    return v;
+  };
   float best1 = 1e30f, best2 = 1e30f;
   int b_t1 = c.tile1, b_t2 = c.tile2, b_k1 = c.kchunk1, b_k2 = c.kchunk2;
   int rc = CHL_OK;
-  for (int t = 0; t < ntiles && rc == CHL_OK; t++) {
-    for (int kc : chunks) {
-      if (kc > 2 * nz1 && kc != chunks.front()) continue;
-      const int k1 = std::min(kc, nz1);
-      float ms     = 0;
-      for (int rep = 0; rep < 2 && rc == CHL_OK; rep++) {  // rep 0 warms up
-        if (hipMemcpyAsync(S, U, bytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) rc = CHL_ERR_HIP;
-        (void)hipEventRecord(e0, h->stream);
-        for (int s = 0; s < steps && rc == CHL_OK; s++) rc = LaunchStage1(h, a, t, k1);
-        (void)hipEventRecord(e1, h->stream);
-        (void)hipEventSynchronize(e1);
-        (void)hipEventElapsedTime(&ms, e0, e1);
-      }
-      if (ms < best1) best1 = ms, b_t1 = t, b_k1 = k1;
+  for (const auto &[t, k1] : shapes(c.tile1, c.kchunk1, nz1)) {
+    float ms = 0;
+    for (int rep = 0; rep < 2 && rc == CHL_OK; rep++) {  // rep 0 warms up
+      if (hipMemcpyAsync(S, U, bytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) rc = CHL_ERR_HIP;
+      (void)hipEventRecord(e0, h->stream);
+      for (int s = 0; s < steps && rc == CHL_OK; s++) rc = LaunchStage1(h, a, t, k1);
+      (void)hipEventRecord(e1, h->stream);
+      (void)hipEventSynchronize(e1);
+      (void)hipEventElapsedTime(&ms, e0, e1);
     }
+    if (ms < best1) best1 = ms, b_t1 = t, b_k1 = k1;
   }
-  for (int t = 0; t < ntiles && rc == CHL_OK; t++) {
-    for (int kc : chunks) {
-      if (kc > 2 * nz2 && kc != chunks.front()) continue;
-      const int k2 = std::min(kc, nz2);
-      float ms     = 0;
-      for (int rep = 0; rep < 2 && rc == CHL_OK; rep++) {
-        if (hipMemcpyAsync(S, U, bytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) rc = CHL_ERR_HIP;
-        if (rc == CHL_OK) rc = LaunchStage1(h, a, b_t1, b_k1);
-        (void)hipEventRecord(e0, h->stream);
-        for (int s = 0; s < steps && rc == CHL_OK; s++) rc = LaunchStage2(h, a, t, k2);
-        (void)hipEventRecord(e1, h->stream);
-        (void)hipEventSynchronize(e1);
-        (void)hipEventElapsedTime(&ms, e0, e1);
-      }
-      if (ms < best2) best2 = ms, b_t2 = t, b_k2 = k2;
+  for (const auto &[t, k2] : shapes(c.tile2, c.kchunk2, nz2)) {
+    float ms = 0;
+    for (int rep = 0; rep < 2 && rc == CHL_OK; rep++) {
+      if (hipMemcpyAsync(S, U, bytes, hipMemcpyDeviceToDevice, h->stream) != hipSuccess) rc = CHL_ERR_HIP;
+      if (rc == CHL_OK) rc = LaunchStage1(h, a, b_t1, b_k1);
+      (void)hipEventRecord(e0, h->stream);
+      for (int s = 0; s < steps && rc == CHL_OK; s++) rc = LaunchStage2(h, a, t, k2);
+      (void)hipEventRecord(e1, h->stream);
+      (void)hipEventSynchronize(e1);
+      (void)hipEventElapsedTime(&ms, e0, e1);
     }
+    if (ms < best2) best2 = ms, b_t2 = t, b_k2 = k2;
   }
   (void)hipStreamSynchronize(h->stream);
   (void)hipEventDestroy(e0);

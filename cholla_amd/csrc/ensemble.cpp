@@ -8,6 +8,7 @@
 #include <limits>
 #include <random>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/cholla_amd.h"
@@ -663,7 +664,6 @@ int chl_ensemble_autotune(chl_ensemble *e, int steps, chl_ensemble_config *chose
   // one clock step so the boxes carry a non-zero dt
   if (rc == CHL_OK && chl::LaunchEnsembleClock(e->clk, e->box, e->n, kCfl, e->head, e->stream) != hipSuccess)
     rc = Fail(CHL_ERR_HIP, "clock launch failed");
-  const int chunks[] = {8, 16, 32, 64};
   // split launch: stage 1 then stage 2, each on its own
   chl_ensemble_config sc = orig;
   sc.launch              = CHL_LAUNCH_SPLIT;
@@ -673,24 +673,32 @@ int chl_ensemble_autotune(chl_ensemble *e, int steps, chl_ensemble_config *chose
                       orig.reconstruction == CHL_RECON_PLMP || orig.reconstruction == CHL_RECON_PPMP;
   const int ntiles = orig.dual_energy || narrow ? chl::kNumDeTiles : chl::kNumTiles;
   if (narrow) sc.tile1 = std::min(sc.tile1, chl::kNumDeTiles - 1), sc.tile2 = std::min(sc.tile2, chl::kNumDeTiles - 1);
-  for (int t = 0; t < ntiles && rc == CHL_OK; t++)
-    for (int kc : chunks) {
-      chl_ensemble_config c = sc;
-      c.tile1 = t, c.kchunk1 = kc;
-      float ms = 0;
-      if ((rc = plan(c)) != CHL_OK) break;
-      if ((rc = timed([&] { return EnqueueStage(e, 1); }, &ms)) != CHL_OK) break;
-      if (ms < b1) b1 = ms, sc.tile1 = t, sc.kchunk1 = kc;
-    }
-  for (int t = 0; t < ntiles && rc == CHL_OK; t++)
-    for (int kc : chunks) {
-      chl_ensemble_config c = sc;
-      c.tile2 = t, c.kchunk2 = kc;
-      float ms = 0;
-      if ((rc = plan(c)) != CHL_OK) break;
-      if ((rc = timed([&] { return EnqueueStage(e, 2); }, &ms)) != CHL_OK) break;
-      if (ms < b2) b2 = ms, sc.tile2 = t, sc.kchunk2 = kc;
-    }
+  // the split launch's shape in hand (the rule's z-chunks may be shorter), then the tiles and chunks
+  auto shapes = [&](int tile, int kchunk) {
+    std::vector<std::pair<int, int>> v;
+    if (orig.launch == CHL_LAUNCH_SPLIT) v.push_back({tile, kchunk});
+    for (int t = 0; t < ntiles; t++)
+      for (int kc : {8, 16, 32, 64}) v.push_back({t, kc});
+    return v;
+  };
+  for (const auto &[t, kc] : shapes(orig.tile1, orig.kchunk1)) {
+    if (rc != CHL_OK) break;
+    chl_ensemble_config c = sc;
+    c.tile1 = t, c.kchunk1 = kc;
+    float ms = 0;
+    if ((rc = plan(c)) != CHL_OK) break;
+    if ((rc = timed([&] { return EnqueueStage(e, 1); }, &ms)) != CHL_OK) break;
+    if (ms < b1) b1 = ms, sc.tile1 = t, sc.kchunk1 = kc;
+  }
+  for (const auto &[t, kc] : shapes(orig.tile2, orig.kchunk2)) {
+    if (rc != CHL_OK) break;
+    chl_ensemble_config c = sc;
+    c.tile2 = t, c.kchunk2 = kc;
+    float ms = 0;
+    if ((rc = plan(c)) != CHL_OK) break;
+    if ((rc = timed([&] { return EnqueueStage(e, 2); }, &ms)) != CHL_OK) break;
+    if (ms < b2) b2 = ms, sc.tile2 = t, sc.kchunk2 = kc;
+  }
   if (rc == CHL_OK && (rc = plan(sc)) == CHL_OK) {
     float ms = 0;
     rc = timed([&] { return EnqueueStep(e); }, &ms);

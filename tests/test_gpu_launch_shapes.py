@@ -137,3 +137,26 @@ def test_mixed_stage1_wide_tiles(dims, wide):
         hy.run(D, *w, G, 0.0, 1e30, 2)
         out.append(D.download())
     assert np.array_equal(out[0], out[1])
+
+
+def test_autotune_keeps_a_faster_picked_shape():
+    """The shapes in hand are among the autotuner's candidates: on a 32^3 box the picked z-chunks
+    of one plane run 3-4 times faster than its own list's 8 to 128, and an ensemble's likewise
+    (a quarter more).  The bar is half the former factor, for the noise of single launches."""
+    ng, dims = 4, (32, 32, 32)
+    U, n = rough_state(dims, ng, 8)
+    w = [1.0 / v for v in dims]
+    D = chl.DeviceArray.from_host(U)
+    hy = chl.Hydro(*n, ng, chl.RECON_PLMC, chl.PREC_FP64_EXACT)
+    hy.kernel_times(D, *w, G, 2)
+    picked = min(sum(hy.kernel_times(D, *w, G, 5)[:2]) for _ in range(4))
+    hy.autotune(D, *w, G)
+    tuned = min(sum(hy.kernel_times(D, *w, G, 5)[:2]) for _ in range(4))
+    assert tuned <= 1.75 * picked, (tuned, picked)
+    ens = chl.Ensemble([n] * 2, ng, chl.RECON_PPMC, chl.PREC_MIXED)
+    states = [chl.DeviceArray.from_host(U) for _ in range(2)]
+    ens.bind(states, [w] * 2)
+    ens.start(G)
+    chunks = ens.config().kchunk1, ens.config().kchunk2
+    cfg = ens.autotune(4)
+    assert max(chunks) < 8 and (cfg.launch == chl.LAUNCH_PERSISTENT or min(cfg.kchunk1, cfg.kchunk2) < 8)
