@@ -395,9 +395,15 @@ size_t chl_capi::HalfStepBytes(const chl_hydro_config &c, size_t *w_main)
 //            its wider rows fit the box (mixed: 300x212x190 289 against 326 us, 512^3 3.12
 //            against 3.30 ms; 200x180x160, a quarter of whose lanes it would idle, 173 against
 //            169 us), which the narrow kernels do not have; stage 2: 16x16,
-//            and 32x16 in the FP64 forms where it rounds better (with PLMC it needs 5 % less:
-//            KH 256^3 1.89 against 2.09 ms), or 16x8 where those leave CUs idle (32^3, PPMC,
-//            fast form: 27 against 28 us), which the narrow kernels do not have
+//            and 32x16 in the FP64 forms where it rounds better, which the narrow kernels do not
+//            have.  With PLMC 32x16 needs 5 % less (KH 256^3 1.89 against 2.09 ms), but 10 % more
+//            while 16x16 leaves a workgroup its CU (256 of them: 64x32x32 exact 25.8 against
+//            23.3 us).  With PPMC boxes of up to 256 workgroups of 16x8 take those, which measure
+//            as 16x16 does (8^3 to 32^3: within 0.5 us of 24 and 31); counted as one per CU they
+//            are not taken where they would share one (64x32x32: 41.5 against 32.3 us)
+//            The HLL, Roe and exact solvers, PCM, PLMP, PPMP, dual energy and gravity follow the
+//            same rule: over 32^3 to 256x192x160 every one of their steps is shorter than on the
+//            former 32x8 tiles and 32-plane chunks, by 13 % (exact solver, the largest) to 20 times
 //   caps     stage 1 loses to its z planes leaving the L2 past 8 (FP64) or 16 planes; stage 2
 //            past 32, with dual energy past 8
 void chl_capi::PickLaunchShape(int stage, int precision, int reconstruction, bool dual_energy, bool narrow,
@@ -428,7 +434,8 @@ void chl_capi::PickLaunchShape(int stage, int precision, int reconstruction, boo
       for (const StageExtent &b : boxes)
         groups += double(chl::CeilDiv(b.x, s.tx)) * chl::CeilDiv(b.y, s.ty) * chl::CeilDiv(b.z, std::min(k, b.z));
       const double rounds = groups <= 4 * slots ? std::ceil(groups / slots) : groups / slots + 0.5;
-      const double cost   = weight * rounds * (k + c0);
+      const double alone  = all && t == 1 && reconstruction == CHL_RECON_PLMC && groups <= cus ? 0.9 : 1.0;
+      const double cost   = alone * weight * rounds * (k + c0);
       if (cost < best) best = cost, best_t = t, best_k = k;
       if (kchunk > 0) break;
     }

@@ -160,3 +160,14 @@ def test_autotune_keeps_a_faster_picked_shape():
     chunks = ens.config().kchunk1, ens.config().kchunk2
     cfg = ens.autotune(4)
     assert max(chunks) < 8 and (cfg.launch == chl.LAUNCH_PERSISTENT or min(cfg.kchunk1, cfg.kchunk2) < 8)
+
+
+@pytest.mark.parametrize("dims,tile", [((8, 8, 8), 1), ((32, 32, 32), 1), ((64, 32, 32), 1), ((40, 40, 40), 4),
+                                       ((128, 128, 128), 4)])
+def test_plmc_takes_wide_tiles_only_where_narrow_ones_share_a_cu(dims, tile):
+    """Stage 2 in FP64 with PLMC: 16x16 tiles while their workgroups are at most one per CU (256),
+    where they measure 10-15 % shorter than 32x16."""
+    for precision in (chl.PREC_FP64_EXACT, chl.PREC_FP64):
+        c = chl.Hydro(*(v + 6 for v in dims), 3, chl.RECON_PLMC, precision).config()
+        assert c.tile2 == tile
+        assert tile == 4 or np.prod([-(-v // 16) for v in dims[:2]]) * -(-dims[2] // c.kchunk2) <= 256
