@@ -1013,9 +1013,61 @@ __device__ __forceinline__ RState<typename P::T> RStateFromPrim(const Prim<typen
   }
 }
 
+// The end of Calculate_HLLC_Fluxes_CUDA (hllc_cuda.cu:174-303) from the signal speeds on: both
+// sides' fluxes and star states averaged with |Sm|.  FP64 only.
+template <class P, bool DE>
+__device__ __forceinline__ Cons<typename P::T> HllcAverage(const RState<typename P::T> &l, const RState<typename P::T> &r,
+                                                           typename P::T Sl, typename P::T Sr, typename P::T *fge)
+{
+  using T = typename P::T;
+  static_assert(!SplitPressure<P>, "the split-pressure form takes one side's star state");
+  // H-correction hook with etah = 0 (hllc_cuda.cu:52,174-175)
+  Sl = ((Sl < T(0)) ? T(-1) : T(1)) * Fmax(Fabs(Sl), T(0));
+  Sr = ((Sr < T(0)) ? T(-1) : T(1)) * Fmax(Fabs(Sr), T(0));
+
+  Cons<T> fl{l.mx, l.mx * l.vx + l.p, l.my * l.vx, l.mz * l.vx, (l.E + l.p) * l.vx};
+  Cons<T> fr{r.mx, r.mx * r.vx + r.p, r.my * r.vx, r.mz * r.vx, (r.E + r.p) * r.vx};
+  T f_ge_l = T(0), f_ge_r = T(0);
+  if constexpr (DE) f_ge_l = l.dge * l.vx, f_ge_r = r.dge * r.vx;
+  if (Sl > T(0.0)) {
+    if constexpr (DE) *fge = f_ge_l;
+    return fl;
+  }
+  if (Sr < T(0.0)) {
+    if constexpr (DE) *fge = f_ge_r;
+    return fr;
+  }
+
+  T Sm = Div1<P>(r.d * r.vx * (Sr - r.vx) - l.d * l.vx * (Sl - l.vx) + l.p - r.p,
+                 r.d * (Sr - r.vx) - l.d * (Sl - l.vx));
+  T ps      = l.d * (l.vx - Sl) * (l.vx - Sm) + l.p;  // star pressure
+  T inv_lsm = Rcp<P>(Sl - Sm), inv_rsm = Rcp<P>(Sr - Sm);
+  T dls     = Div<P>(l.d * (Sl - l.vx), Sl - Sm, inv_lsm);
+  T mxls    = Div<P>(l.mx * (Sl - l.vx) + ps - l.p, Sl - Sm, inv_lsm);
+  T myls = dls * l.vy, mzls = dls * l.vz;
+  T Els  = Div<P>(l.E * (Sl - l.vx) - l.p * l.vx + ps * Sm, Sl - Sm, inv_lsm);
+  T drs  = Div<P>(r.d * (Sr - r.vx), Sr - Sm, inv_rsm);
+  T mxrs = Div<P>(r.mx * (Sr - r.vx) + ps - r.p, Sr - Sm, inv_rsm);
+  T myrs = drs * r.vy, mzrs = drs * r.vz;
+  T Ers  = Div<P>(r.E * (Sr - r.vx) - r.p * r.vx + ps * Sm, Sr - Sm, inv_rsm);
+  T aSm  = Fabs(Sm);
+  Cons<T> f;
+  f.d  = T(0.5) * (fl.d + fr.d + (Sr - aSm) * drs + (Sl + aSm) * dls - Sl * l.d - Sr * r.d);
+  f.mx = T(0.5) * (fl.mx + fr.mx + (Sr - aSm) * mxrs + (Sl + aSm) * mxls - Sl * l.mx - Sr * r.mx);
+  f.my = T(0.5) * (fl.my + fr.my + (Sr - aSm) * myrs + (Sl + aSm) * myls - Sl * l.my - Sr * r.my);
+  f.mz = T(0.5) * (fl.mz + fr.mz + (Sr - aSm) * mzrs + (Sl + aSm) * mzls - Sl * l.mz - Sr * r.mz);
+  f.E  = T(0.5) * (fl.E + fr.E + (Sr - aSm) * Ers + (Sl + aSm) * Els - Sl * l.E - Sr * r.E);
+  if constexpr (DE) {
+    T gel = Div<P>(l.dge, l.d, l.inv_d), ger = Div<P>(r.dge, r.d, r.inv_d);
+    T gels = dls * gel, gers = drs * ger;
+    *fge   = T(0.5) * (f_ge_l + f_ge_r + (Sr - aSm) * gers + (Sl + aSm) * gels - Sl * l.dge - Sr * r.dge);
+  }
+  return f;
+}
+
 // Calculate_HLLC_Fluxes_CUDA body, src/riemann_solvers/hllc_cuda.cu:141-305 (etah = 0).
 // Returns the flux in rotated order; with dual energy the GasEnergy flux goes to
-// *fge (hllc_cuda.cu:183-198, 218-235, 251-303).
+// *fge (hllc_cuda.cu:183-198, 218-235, 251-303).  HALF: a face of the half step.
 template <class P, bool DE = false, bool HALF = false>
 __device__ __forceinline__ Cons<typename P::T> Hllc(const RState<typename P::T> &l, const RState<typename P::T> &r,
                                                     typename P::T gamma, typename P::T *fge = nullptr)
@@ -1051,9 +1103,9 @@ __device__ __forceinline__ Cons<typename P::T> Hllc(const RState<typename P::T> 
   }
   T Sl  = Fmin(lambda_m, l.vx - cfl);
   T Sr  = Fmax(lambda_p, r.vx + cfr);
-  // momentum-flux pressures (the pressures themselves outside the split-pressure form)
-  const T pml = MomP<P>(l), pmr = MomP<P>(r);
-  if constexpr (P::kId == PolicyMixed::kId || (!P::kExact && !HALF)) {
+  if constexpr (!HALF && !P::kExact) {
+    // momentum-flux pressures (the pressures themselves outside the split-pressure form)
+    const T pml = MomP<P>(l), pmr = MomP<P>(r);
     // The flux of the one state on the face.  The reference averages both sides' fluxes and
     // star states with |Sm|, which in exact arithmetic is the physical flux of the left star
     // state for Sm >= 0 and of the right one below (jump conditions across Sl, Sm, Sr): the
@@ -1086,50 +1138,9 @@ __device__ __forceinline__ Cons<typename P::T> Hllc(const RState<typename P::T> 
     f.E  = (sup ? E + p : Es + ps) * u;
     if constexpr (DE) *fge = mass * (lf ? l.dge * l.inv_d : r.dge * r.inv_d);
     return f;
+  } else {
+    return HllcAverage<P, DE>(l, r, Sl, Sr, fge);
   }
-  // H-correction hook with etah = 0 (hllc_cuda.cu:52,174-175)
-  Sl = ((Sl < T(0)) ? T(-1) : T(1)) * Fmax(Fabs(Sl), T(0));
-  Sr = ((Sr < T(0)) ? T(-1) : T(1)) * Fmax(Fabs(Sr), T(0));
-
-  Cons<T> fl{l.mx, l.mx * l.vx + pml, l.my * l.vx, l.mz * l.vx, (l.E + l.p) * l.vx};
-  Cons<T> fr{r.mx, r.mx * r.vx + pmr, r.my * r.vx, r.mz * r.vx, (r.E + r.p) * r.vx};
-  T f_ge_l = T(0), f_ge_r = T(0);
-  if constexpr (DE) f_ge_l = l.dge * l.vx, f_ge_r = r.dge * r.vx;
-  if (Sl > T(0.0)) {
-    if constexpr (DE) *fge = f_ge_l;
-    return fl;
-  }
-  if (Sr < T(0.0)) {
-    if constexpr (DE) *fge = f_ge_r;
-    return fr;
-  }
-
-  T Sm = Div1<P>(r.d * r.vx * (Sr - r.vx) - l.d * l.vx * (Sl - l.vx) + pml - pmr,
-                 r.d * (Sr - r.vx) - l.d * (Sl - l.vx));
-  T psm     = l.d * (l.vx - Sl) * (l.vx - Sm) + pml;  // star pressure (less p0 when split)
-  T ps      = SplitPressure<P> ? psm + l.p0 : psm;
-  T inv_lsm = Rcp<P>(Sl - Sm), inv_rsm = Rcp<P>(Sr - Sm);
-  T dls     = Div<P>(l.d * (Sl - l.vx), Sl - Sm, inv_lsm);
-  T mxls    = Div<P>(l.mx * (Sl - l.vx) + psm - pml, Sl - Sm, inv_lsm);
-  T myls = dls * l.vy, mzls = dls * l.vz;
-  T Els  = Div<P>(l.E * (Sl - l.vx) - l.p * l.vx + ps * Sm, Sl - Sm, inv_lsm);
-  T drs  = Div<P>(r.d * (Sr - r.vx), Sr - Sm, inv_rsm);
-  T mxrs = Div<P>(r.mx * (Sr - r.vx) + psm - pmr, Sr - Sm, inv_rsm);
-  T myrs = drs * r.vy, mzrs = drs * r.vz;
-  T Ers  = Div<P>(r.E * (Sr - r.vx) - r.p * r.vx + ps * Sm, Sr - Sm, inv_rsm);
-  T aSm  = Fabs(Sm);
-  Cons<T> f;
-  f.d  = T(0.5) * (fl.d + fr.d + (Sr - aSm) * drs + (Sl + aSm) * dls - Sl * l.d - Sr * r.d);
-  f.mx = T(0.5) * (fl.mx + fr.mx + (Sr - aSm) * mxrs + (Sl + aSm) * mxls - Sl * l.mx - Sr * r.mx);
-  f.my = T(0.5) * (fl.my + fr.my + (Sr - aSm) * myrs + (Sl + aSm) * myls - Sl * l.my - Sr * r.my);
-  f.mz = T(0.5) * (fl.mz + fr.mz + (Sr - aSm) * mzrs + (Sl + aSm) * mzls - Sl * l.mz - Sr * r.mz);
-  f.E  = T(0.5) * (fl.E + fr.E + (Sr - aSm) * Ers + (Sl + aSm) * Els - Sl * l.E - Sr * r.E);
-  if constexpr (DE) {
-    T gel = Div<P>(l.dge, l.d, l.inv_d), ger = Div<P>(r.dge, r.d, r.inv_d);
-    T gels = dls * gel, gers = drs * ger;
-    *fge   = T(0.5) * (f_ge_l + f_ge_r + (Sr - aSm) * gers + (Sl + aSm) * gels - Sl * l.dge - Sr * r.dge);
-  }
-  return f;
 }
 
 // Calculate_HLL_Fluxes_CUDA body, src/riemann_solvers/hll_cuda.cu:141-266: Davis wave
@@ -1412,7 +1423,8 @@ __device__ __forceinline__ Cons<typename P::T> RiemannFlux(const RState<typename
   } else if constexpr (P::kSolver == kRiemannExact) {
     return ExactFlux<P, DE>(l, r, gamma, fge);
   } else {
-    return Hllc<P, DE, HALF>(l, r, gamma, fge);
+    // the half step's faces differ in the fast FP64 form alone
+    return Hllc<P, DE, HALF && P::kId == PolicyFast::kId>(l, r, gamma, fge);
   }
 }
 

@@ -5,11 +5,13 @@ import numpy as np
 import pytest
 
 import cholla_amd as chl
-from helpers import check_fp64, check_mixed, interior, rel_l1
+from helpers import FIELD_NAMES, check_fp64, check_mixed, interior, rel_l1
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
 G, NG, DIMS = 5 / 3, 4, (40, 7, 6)
+STREAMS = [((1, 3, 1), (0.5, 3, 0.4)), ((1, -3, 1), (0.5, -3, 0.4)), ((1, 0.4, 1), (0.3, 0.4, 0.9)),
+           ((1, -0.4, 1), (0.3, -0.4, 0.9)), ((1, 1.5, 1), (1, -1.5, 1)), ((1, -0.5, 1), (1, 0.5, 1))]
 RECON = {orc.PLMC: chl.RECON_PLMC, orc.PPMC: chl.RECON_PPMC}
 
 
@@ -26,18 +28,16 @@ def halves(left, right, noise, seed=9):
     return U, (nx, ny, nz)
 
 
-def step(U, dims, recon, precision, steps):
+def step(U, dims, recon, precision, steps, dual_energy=False):
     D = chl.DeviceArray.from_host(U)
-    hy = chl.Hydro(*dims, NG, RECON[recon], precision)
+    hy = chl.Hydro(*dims, NG, RECON[recon], precision, dual_energy=dual_energy)
     hy.run(D, *[1.0 / v for v in DIMS], G, 0.0, 1e30, steps)
     return D.download()
 
 
 @pytest.mark.parametrize("precision", [chl.PREC_FP64, chl.PREC_MIXED])
 @pytest.mark.parametrize("recon", [orc.PLMC, orc.PPMC])
-@pytest.mark.parametrize("left,right", [((1, 3, 1), (0.5, 3, 0.4)), ((1, -3, 1), (0.5, -3, 0.4)),
-                                        ((1, 0.4, 1), (0.3, 0.4, 0.9)), ((1, -0.4, 1), (0.3, -0.4, 0.9)),
-                                        ((1, 1.5, 1), (1, -1.5, 1)), ((1, -0.5, 1), (1, 0.5, 1))])
+@pytest.mark.parametrize("left,right", STREAMS)
 def test_every_selection_within_the_forms_bars(left, right, recon, precision):
     U, dims = halves(left, right, 0.05)
     A = U.copy()
@@ -45,6 +45,23 @@ def test_every_selection_within_the_forms_bars(left, right, recon, precision):
     B = step(U, dims, recon, precision, 2)
     l1 = [rel_l1(b, a) for b, a in zip(interior(B, 5, *dims, NG), interior(A, 5, *dims, NG))]
     (check_fp64 if precision == chl.PREC_FP64 else check_mixed)(l1)
+
+
+@pytest.mark.parametrize("precision", [chl.PREC_FP64, chl.PREC_MIXED])
+@pytest.mark.parametrize("recon", [orc.PLMC, orc.PPMC])
+@pytest.mark.parametrize("left,right", STREAMS)
+def test_dual_energy_faces_within_the_forms_bars(left, right, recon, precision):
+    """The GasEnergy flux of each selection, with the gas energy well above the switch's 1e-3 of the
+    total (the supersonic streams' internal energy is 5-30 % of it), so that no cell changes side."""
+    U, dims = halves(left, right, 0.05)
+    q = U.reshape(5, -1)
+    U = np.concatenate([U, q[4] - 0.5 * (q[1] ** 2 + q[2] ** 2 + q[3] ** 2) / q[0]])
+    A = U.copy()
+    orc.run(A, *dims, NG, 6, *[1.0 / v for v in DIMS], G, recon, [1] * 6, 0.0, 1e30, 2, dual_energy_on=True)
+    B = step(U, dims, recon, precision, 2, dual_energy=True)
+    l1 = [rel_l1(b, a) for b, a in zip(interior(B, 6, *dims, NG), interior(A, 6, *dims, NG))]
+    names = tuple(FIELD_NAMES[:5]) + ("GasEnergy",)
+    (check_fp64 if precision == chl.PREC_FP64 else check_mixed)(l1, names=names)
 
 
 @pytest.mark.parametrize("precision", [chl.PREC_FP64, chl.PREC_MIXED])
