@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 import cholla_amd as chl
+from helpers import check_mixed, interior, rel_l1
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -133,3 +134,20 @@ def test_fp64_form_keeps_tails_bounded(vz):
     assert np.isfinite(out).all()
     slack = 1e-12 * vz + 20 * 5e-324
     assert out[3].min() >= 0.5 * vz - slack and out[3].max() <= vz + slack
+
+
+@pytest.mark.parametrize("recon", [orc.PLMC, orc.PPMC])
+@pytest.mark.parametrize("d_scale,p_scale", [(2.0 ** 60, 2.0 ** 50), (2.0 ** -55, 2.0 ** -55), (2.0 ** -40, 2.0 ** 30)])
+def test_mixed_form_far_from_one(recon, d_scale, p_scale):
+    """The FP32 quotients where products of two slopes are far from 1 (1e-35 to 1e35, normal in FP32):
+    the mixed form's bar on every field that moves."""
+    n, ng, g = 16, 4, 5 / 3
+    U, N = scaled_box(n, ng, d_scale, p_scale, 0.0)
+    h = 1.0 / n
+    A = U.copy()
+    orc.run(A, N, N, N, ng, 5, h, h, h, g, recon, [1] * 6, 0.0, 1e300, 3)
+    D = chl.DeviceArray.from_host(U)
+    hy = chl.Hydro(N, N, N, ng, RECON[recon], chl.PREC_MIXED)
+    hy.run(D, h, h, h, g, 0.0, 1e300, 3)
+    a, b = (interior(q, 5, N, N, N, ng) for q in (A, D.download()))
+    check_mixed([rel_l1(b[f], a[f]) for f in (0, 1, 2, 4)], names=["density", "momentum_x", "momentum_y", "Energy"])

@@ -27,7 +27,8 @@ def rough_state(dims, ng, seed, fields=5):
     return U, (nx, ny, nz)
 
 
-# the smallest periodic box of 4 ghost cells; one plane per workgroup; a remainder in every axis; more than four rounds
+# the smallest periodic box of 4 ghost cells, remainders in every axis, one to four planes per workgroup; each is
+# under one round of workgroups (test_picked_shape_of_many_rounds has the others)
 SIZES = [(4, 5, 4), (33, 17, 5), (24, 24, 24), (70, 9, 50), (130, 66, 36)]
 
 
@@ -61,6 +62,32 @@ def test_picked_shape_matches_explicit(dims, precision):
     assert np.abs(out[0] - out[1]).max() <= (0 if precision == chl.PREC_FP64 else 4e-16 * np.abs(out[1]).max())
 
 
+TILES = [(32, 8), (16, 16), (64, 4), (16, 8), (32, 16)]
+
+
+@pytest.mark.parametrize("precision", [chl.PREC_FP64, chl.PREC_MIXED])
+def test_picked_shape_of_many_rounds(precision):
+    """A long thin box of more than four rounds of workgroups in both stages, whose picked chunks are
+    long: alike with explicit tiles and chunks."""
+    ng, dims = 4, (33, 33, 4100)
+    U, n = rough_state(dims, ng, 5)
+    w = [1.0 / v for v in dims]
+    out = []
+    for kw in ({}, dict(tile1=0, tile2=0, kchunk1=32, kchunk2=32)):
+        D = chl.DeviceArray.from_host(U)
+        hy = chl.Hydro(*n, ng, chl.RECON_PPMC, precision, **kw)
+        if not kw:
+            c = hy.config()
+            waves = {1: 4, 2: 3 if precision == chl.PREC_MIXED else 2}  # per SIMD of 256 CUs
+            for stage, tile, k, ext in ((1, c.tile1, c.kchunk1, [v + 6 for v in dims]), (2, c.tile2, c.kchunk2, dims)):
+                tx, ty = TILES[tile]
+                groups = -(-ext[0] // tx) * -(-ext[1] // ty) * -(-ext[2] // k)
+                assert k >= 8 and groups > 4 * 256 * waves[stage] * 256 // (tx * ty), (stage, tile, k, groups)
+        hy.run(D, *w, G, 0.0, 1e30, 1)
+        out.append(D.download())
+    assert np.abs(out[0] - out[1]).max() <= (0 if precision == chl.PREC_FP64 else 4e-16 * np.abs(out[1]).max())
+
+
 def test_picked_ensemble_shape_matches_single_boxes():
     ng, dims = 4, [(8, 8, 8), (20, 12, 40), (33, 33, 33)]
     states, ref = [], []
@@ -79,9 +106,12 @@ def test_picked_ensemble_shape_matches_single_boxes():
 
 
 @pytest.mark.parametrize("recon,ng", [(orc.MHD_PLMC, 4), (orc.MHD_PPMC, 5)])
-@pytest.mark.parametrize("dims", [(5, 6, 5), (60, 9, 7), (35, 34, 70)])
+@pytest.mark.parametrize("dims", [(5, 6, 5), (60, 9, 7), (35, 34, 70), (33, 9, 8300)])
 def test_mhd_chunks_match_oracle(dims, recon, ng):
-    # a chunk of one plane, remainders along each march, several rounds
+    # a chunk of one plane, remainders along each march, most of a round, more than four rounds at
+    # the longest chunks (4 columns of tiles x 519 chunks of 16 planes over 512 slots)
+    if recon == orc.MHD_PPMC and dims[2] > 1000:
+        pytest.skip("the chunk rule does not depend on the reconstruction")
     U0 = chl.ic_orszag_tang(8, ng, G, seed=5)
     nx, ny, nz = (v + 2 * ng for v in dims)
     V = U0.reshape(8, *(8 + 2 * ng,) * 3)[:, ng:-ng, ng:-ng, ng:-ng]
@@ -104,9 +134,9 @@ def test_mhd_chunks_match_oracle(dims, recon, ng):
     assert np.isfinite(A).all() and np.array_equal(D.download(), A)
 
 
-@pytest.mark.parametrize("dims", [(4, 5, 4), (65, 5, 9), (63, 33, 17), (96, 40, 44)])
+@pytest.mark.parametrize("dims", [(4, 4, 4), (4, 5, 4), (65, 5, 9), (63, 33, 17), (96, 40, 44)])
 def test_de_sync_columns_match_oracle(dims):
-    # columns of 64 x 4 with remainders in x and y, one workgroup, one and several planes each
+    # columns of 64 x 4: one workgroup, then remainders in x and y, and 4 to 10 planes each
     ng = 4
     U5, (nx, ny, nz) = rough_state(dims, ng, 11)
     U = np.concatenate([U5, np.zeros(nx * ny * nz)])
