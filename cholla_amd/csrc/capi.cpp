@@ -390,13 +390,13 @@ size_t chl_capi::HalfStepBytes(const chl_hydro_config &c, size_t *w_main)
 // tile and z-chunk on boxes of 32^3 to 384^3 the pick is 1-5 % off in the mean and 29 % at
 // worst; the 32-plane chunks of one fixed tile it replaced left a 48^3 box to 12-18 workgroups
 // (stage 1 / 2, PLMC, reference order: 209 / 406 us against 22 / 34) and KH 512^3 (mixed) on
-// stage-2 tiles of 16x8 (10.2 ms against 8.5).
+// stage-2 tiles of 16x8 (8.5 ms against 7.4).
 //   tiles    stage 1: 16x16 (FP64), 32x8 (mixed: KH 256^3 495 against 536 us), or 64x4 where
 //            its wider rows fit the box (mixed: 300x212x190 289 against 326 us, 512^3 3.12
 //            against 3.30 ms; 200x180x160, a quarter of whose lanes it would idle, 173 against
 //            169 us), which the narrow kernels do not have; stage 2: 16x16,
 //            and 32x16 in the FP64 forms where it rounds better, which the narrow kernels do not
-//            have.  With PLMC 32x16 needs 5 % less (KH 256^3 1.89 against 2.09 ms), but 10 % more
+//            have.  With PLMC 32x16 needs less (KH 256^3 exact 1.84 against 2.12 ms), but 10 % more
 //            while 16x16 leaves a workgroup its CU (256 of them: 64x32x32 exact 25.8 against
 //            23.3 us).  With PPMC boxes of up to 256 workgroups of 16x8 take those, which measure
 //            as 16x16 does (8^3 to 32^3: within 0.5 us of 24 and 31); counted as one per CU they

@@ -17,8 +17,8 @@ hipError_t LaunchRepairExact(const StepArgs &a, hipStream_t s) { return LaunchRe
 
 // The side buffer of a density repair next to fused periodic images, one lane per face cell,
 // and in a workgroup of its own the device clock (clk.dti null: no clock).  Neither reads what
-// the other writes, and as two launches each cost a small box its ~4.5 us: a 64x32x32 step
-// 55.6 -> 54.1 us (PLMC, reference order).
+// the other writes, and a launch of its own cost the clock its 1.4 us: a 64x32x32 step 55.6 ->
+// 54.1 us (PLMC, reference order); this launch is the 3.9 us of its side buffer either way.
 __global__ void RepairSideKernel(const double *U, double *side, int nx, int ny, int nz, int ng, StepClock clk)
 {
   if (blockIdx.x + 1 == gridDim.x) {

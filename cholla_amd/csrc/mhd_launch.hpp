@@ -40,7 +40,10 @@ void MhdFlux2Tiles(const mhd::MhdArgs &a, int lo, int hx, int hy, int hz, hipStr
 {
   const unsigned ex = unsigned(hx - lo + 1), ey = unsigned(hy - lo + 1), ez = unsigned(hz - lo + 1);
   auto blocks = [](unsigned t) { return dim3((t + 7) / 8 * 8); };
-  constexpr int kSlots = P::kId == PolicyMixed::kId ? 512 : 256;  // two workgroups per CU, FP64 one
+  // counted as two workgroups per CU in the mixed form and one in FP64, fewer than the registers
+  // admit (3-4 and 1-2).  The chunk so taken costs a step up to 4 % against the best one (64^3,
+  // mixed), under 1 % from 128^3 on
+  constexpr int kSlots = P::kId == PolicyMixed::kId ? 512 : 256;
   const unsigned bx = (ex + 63) / 64;
   const unsigned ky = unsigned(MhdChunk(long(bx) * ((ez + 3) / 4), int(ey), kSlots, 1.0, 16));
   const unsigned kz = unsigned(MhdChunk(long(bx) * ((ey + 3) / 4), int(ez), kSlots, 1.0, 16));

@@ -10,9 +10,10 @@
 // rows of 32 consecutive z.  Bound by HBM on large fields: 16 bytes per cell.  Grid rows start
 // n_ghost cells into a line, so neighbouring tiles share a line at each row end; the 64 x 32
 // tiles go out in XCD-contiguous order, x fastest, which keeps both halves of that line in one
-// L2 (two XCDs each fetched it, or wrote its half through).  A 256^3 field: unpack 84.7 -> 61.9
-// us, pack 54.7 -> 54.8; 300x212x190: pack 57.8 -> 42.4 us, unpack 56.4 -> 44.0 (4.3-4.9 TB/s;
-// a plain copy reaches 4.8), against 32x32 tiles in dispatch order.
+// L2 (two XCDs each fetched it, or wrote its half through).  Launched over and over, a 256^3
+// field: unpack 84.7 -> 61.9 us, pack 54.7 -> 54.8; 300x212x190: pack 57.8 -> 42.4 us, unpack 56.4
+// -> 44.0 (4.3-4.9 TB/s; a plain copy reaches 4.8), against 32x32 tiles in dispatch order.  In
+// passes of five packs and five unpacks of a 256^3 state they take 73 and 52 us.
 #include <hip/hip_runtime.h>
 
 #include <cstddef>

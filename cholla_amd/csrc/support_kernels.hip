@@ -178,8 +178,10 @@ __device__ __forceinline__ void BlockMaxToGlobal(double v, unsigned long long *o
 
 // The real cells of a 3D box by 64 x 4 (x, y) columns of kz planes per workgroup, for a
 // reduction that ends in one atomic per workgroup: that address takes one every ~14 ns, so about
-// 2048 cells per workgroup and up to 2048 workgroups (371 for a box of 120x88x72, where one per
-// 256 cells spent 3 times longer in the atomics than in the cells).
+// 2048 cells per workgroup and about 2048 workgroups at most (396 for a box of 120x88x72, where one
+// per 256 cells spent 3 times longer in the atomics than in the cells; 2200 for 200^3).  The
+// columns are a lower limit: 4096 for 1024x1024x64; and a box a little over a multiple of 64 in x
+// leaves its last column's lanes idle, with fewer cells to the workgroup.
 struct RealColumns {
   int kz, cols_x, cols_y;
   dim3 grid;

@@ -20,8 +20,9 @@ namespace chl
 // (CELLS: up to two) per thread.  Each face is solved and each cell reconstructed once; the
 // unfused stage 2 reconstructs three cells per thread.  What bounds it is the latency of the
 // dependent FP64 chain of a reconstruction and a solve on one or two waves per SIMD.  Sod, 100
-// cells, PLMC, reference order: 26.6 -> 4.5 us a step.  Above 1024 cells the launches spread over
-// the chip and win.
+// cells, PLMC, reference order: 26.6 -> 4.5 us a step.  The limit of 1024 cells is the LDS's (15
+// doubles a cell, 120 of its 160 KB) and two cells a thread, not a crossover: 1024 cells (ghosts
+// included) take 12.3 us a step here, 1025 in the unfused launches 23.6, and 4008 there 24.2.
 constexpr int kLineThreads = 512;
 
 template <class P, int RK, int CELLS>
@@ -210,9 +211,9 @@ hipError_t LaunchVl1dRun(double *U, int n, int ng, int recon, int form, double d
 // half of a workgroup's threads take the x sweep of the tile's cells and half the y sweep, so a
 // thread's chain is one reconstruction and one solve; neighbours exchange through LDS, and the
 // tile's last row and column (and in stage 2 its first) only feed the others.  Periodic boxes
-// write their ghost images from the update.  KH 320x192, PPMC, fast form: stage 2 15.8 us
-// and stage 1 7.7, against 16.8 + 6.5 and 5.5 + 5.8 for the pairs of launches they replace, and
-// no ghost fill (4.4); a step 35 us against 50.
+// write their ghost images from the update.  KH 320x192, PPMC, fast form: stage 2 13.5 us
+// and stage 1 7.6, against 16.8 + 6.5 and 5.5 + 5.8 for the pairs of launches they replaced, and
+// no ghost fill (4.4); a step 33 us against 51.
 
 // Stage 1: PCM states and HLLC on the lower x and y faces of a 32 x 8 tile of cells, the dt/2
 // update of its 31 x 7 cells whose upper faces it holds too (Update_Conserved_Variables_2D_half,
