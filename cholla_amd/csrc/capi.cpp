@@ -337,6 +337,14 @@ int EnqueueRun1d(chl_hydro *h, double *U, double dx, double gamma, int n_steps, 
   return CHL_OK;
 }
 
+// The scratch of a 2D box: the fused step's half state, or the unfused step's half state, 4
+// interface and 2 flux arrays of 6 fields.
+size_t Scratch2d(const chl_hydro_config &c, const chl::GravSpec &grav)
+{
+  const bool fused = chl::Vl2dFusedTakes(c.ny, c.reconstruction, SolverKind(c.riemann), c.dual_energy != 0, grav);
+  return (fused ? 5 : 42) * size_t(c.nx) * c.ny * sizeof(double);
+}
+
 }  // namespace
 
 size_t chl_capi::RepairBytes(const chl_hydro_config &c)
@@ -544,7 +552,7 @@ int chl_hydro_create(const chl_hydro_config *cfg, chl_hydro **out)
   h->num_cu        = p.multiProcessorCount;
   size_t w_main    = 0;
   h->W_bytes       = chl_capi::HalfStepBytes(c, &w_main);
-  if (h->two_d) h->W_bytes = 42 * h->n_cells * sizeof(double);  // half state, 4 interface, 2 flux arrays of 6 fields
+  if (h->two_d) h->W_bytes = Scratch2d(c, h->grav);
   if (h->one_d)  // the 1D integrator's half state is FP64 in every form
     h->W_bytes = std::max(h->W_bytes, (5 + size_t(c.dual_energy)) * h->n_cells * sizeof(double));
   hipError_t e     = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
@@ -758,6 +766,20 @@ int chl_hydro_set_static_gravity(chl_hydro *h, int custom_grav, int x_off, int y
   const bool same = o.id == g.id && o.off[0] == g.off[0] && o.off[1] == g.off[1] && o.off[2] == g.off[2] &&
                     o.bound[0] == g.bound[0] && o.bound[1] == g.bound[1] && o.bound[2] == g.bound[2];
   if (same) return CHL_OK;
+  if (h->two_d && Scratch2d(c, g) > h->W_bytes) {  // the unfused step from here on
+    CHL_HIP(hipStreamSynchronize(h->stream));
+    const size_t bytes = Scratch2d(c, g);
+    (void)hipFree(h->W);
+    hipError_t e = hipMalloc(&h->W, bytes);
+    if (e != hipSuccess) {  // the handle stays as it was, without gravity
+      (void)hipGetLastError();
+      h->W = nullptr;
+      CHL_HIP(hipMalloc(&h->W, h->W_bytes));
+      return Fail(CHL_ERR_HIP, std::string("allocating 2D scratch for gravity: ") + hipGetErrorString(e));
+    }
+    h->W_bytes = bytes;
+    CHL_HIP(hipMemsetAsync(h->W, 0, bytes, h->stream));
+  }
   h->grav = g;
   if (h->graph) {  // the captured step holds the old arguments
     (void)hipGraphExecDestroy(h->graph);

@@ -4,6 +4,7 @@ and 1D in their integrators.  The fields use log, pow, atan2, cos and sin, whose
 differs between the host's libm and the device's math library, so the bar is a per-field
 relative L1 of 1e-12 in the FP64 forms (1e-5 mixed); everything else in the step is
 bit-identical.  Offsets and bounds are non-trivial so the cell positions are checked too."""
+import ctypes
 import sys
 
 import numpy as np
@@ -255,3 +256,39 @@ def test_static_gravity_takes_the_shape_picked_for_its_tiles():
     assert shape(given) == (1, 7)
     given.set_static_gravity(0)
     assert shape(given) == (tile, 7)
+
+
+def free_bytes():
+    """Free device memory, from the HIP runtime the library is linked to."""
+    hip = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(hip).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_2d_scratch_follows_gravity():
+    """A 2D box of the fused step holds its half state alone (5 fields, the unfused step's scratch is
+    42); gravity set after steps of it, and taken off again, gives what a new handle gives."""
+    nx = ny = 2000
+    warm = chl.Hydro(32, 32, 1, 4, chl.RECON_PPMC, chl.PREC_FP64)  # the runtime's own allocations
+    free = free_bytes()
+    big = chl.Hydro(nx, ny, 1, 4, chl.RECON_PPMC, chl.PREC_FP64)
+    assert free - free_bytes() < 10 * nx * ny * 8
+    big.close()
+    warm.close()
+
+    ng, shape = 4, (20, 24)
+    U, (Ny, Nx) = disk_box(shape, ng, seed=12, p0=1.0)  # as above: dt g stays small
+    orc.set_boundaries(U, Nx, Ny, 1, 5, ng, [1, 1, 1, 1, 0, 0])
+    h, off, bnd = 0.1, (2, 3, 0), (-1.0, -1.2, 0.0)
+    D = chl.DeviceArray.from_host(U)
+    hy = chl.Hydro(Nx, Ny, 1, ng, chl.RECON_PPMC, chl.PREC_FP64_EXACT)
+    for grav in (0, 1, 0):
+        start = D.download()
+        hy.set_static_gravity(grav, off, bnd)
+        hy.run(D, h, h, h, G, 0.0, 1e30, 3, use_graph=True)
+        fresh = chl.Hydro(Nx, Ny, 1, ng, chl.RECON_PPMC, chl.PREC_FP64_EXACT)
+        fresh.set_static_gravity(grav, off, bnd)
+        E = chl.DeviceArray.from_host(start)
+        fresh.run(E, h, h, h, G, 0.0, 1e30, 3, use_graph=False)
+        assert np.isfinite(E.download()).all() and np.array_equal(D.download(), E.download()), grav
