@@ -16,6 +16,7 @@
 // passes of five packs and five unpacks of a 256^3 state they take 73 and 52 us.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstddef>
 
 #include "snapshot_kernels.hpp"
@@ -31,17 +32,17 @@ constexpr int kThreads = 256;
 // PACK: grid -> buf (converted to OUT); !PACK: buf -> grid.  (ox, oy, oz) is the grid index of
 // the dataset's first element: n_ghost, or n_ghost - 1 along a magnetic field's own axis
 // (its dataset holds one more face than there are real cells).  TX 64: a linear grid of
-// tiles in XCD-contiguous order; TX 32: the grid's axes are the tiles'.
+// the tiles from `first` on in XCD-contiguous order; TX 32: the grid's axes are the tiles'.
 template <bool PACK, typename OUT, int kTX>
 __global__ void __launch_bounds__(kThreads) SnapshotTileKernel(double *grid, OUT *buf, int nx, int ny, int nxr, int nyr,
                                                               int nzr, int ox, int oy, int oz, unsigned gx,
-                                                              unsigned gz, unsigned tiles)
+                                                              unsigned gz, unsigned first, unsigned tiles)
 {
   __shared__ double t[kTZ][kTX + 1];
   int i0, k0, j;
   if constexpr (kTX == 64) {
-    const unsigned per = (tiles + 7) / 8, q = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((blockIdx.x >> 3) >= per || q >= tiles) return;
+    const unsigned per = (tiles + 7) / 8, n = (blockIdx.x & 7) * per + (blockIdx.x >> 3), q = first + n;
+    if ((blockIdx.x >> 3) >= per || n >= tiles) return;
     i0 = int(q % gx) * kTX, k0 = int(q / gx % gz) * kTZ, j = int(q / (gx * gz));
   } else {
     i0 = int(blockIdx.x) * kTX, k0 = int(blockIdx.y) * kTZ, j = int(blockIdx.z);
@@ -90,13 +91,22 @@ hipError_t Launch(double *grid, OUT *buf, const SnapshotShape &s, hipStream_t st
   const unsigned gz = unsigned((s.nzr + kTZ - 1) / kTZ);
   if (size_t(s.nxr) * s.nyr * s.nzr < kLargeField && s.nyr <= 65535) {
     hipLaunchKernelGGL((SnapshotTileKernel<PACK, OUT, 32>), dim3(unsigned((s.nxr + 31) / 32), gz, unsigned(s.nyr)),
-                       dim3(kThreads), 0, st, grid, buf, s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, 0u, 0u, 0u);
+                       dim3(kThreads), 0, st, grid, buf, s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, 0u, 0u, 0u,
+                       0u);
     return hipGetLastError();
   }
-  const unsigned gx = unsigned((s.nxr + 63) / 64), tiles = gx * gz * unsigned(s.nyr);
-  hipLaunchKernelGGL((SnapshotTileKernel<PACK, OUT, 64>), dim3((tiles + 7) / 8 * 8), dim3(kThreads), 0, st, grid, buf,
-                     s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, gx, gz, tiles);
-  return hipGetLastError();
+  // 2^23 tiles a launch: one of 2^24 has the 2^32 threads that a launch may not reach, which a 2D
+  // field of 32768^2 does
+  constexpr size_t kPerLaunch = size_t(1) << 23;
+  const unsigned gx = unsigned((s.nxr + 63) / 64);
+  const size_t all  = size_t(gx) * gz * s.nyr;
+  for (size_t first = 0; first < all; first += kPerLaunch) {
+    const unsigned tiles = unsigned(std::min(kPerLaunch, all - first));
+    hipLaunchKernelGGL((SnapshotTileKernel<PACK, OUT, 64>), dim3((tiles + 7) / 8 * 8), dim3(kThreads), 0, st, grid,
+                       buf, s.nx, s.ny, s.nxr, s.nyr, s.nzr, s.ox, s.oy, s.oz, gx, gz, unsigned(first), tiles);
+    if (const hipError_t e = hipGetLastError()) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace

@@ -47,3 +47,20 @@ def test_pack_and_unpack_large_fields(dims):
     G = chl.DeviceArray(F.size, np.zeros(F.size))
     chl.check(chl.lib().chl_unpack_real_cells(buf.ptr, G.ptr, *args))
     assert np.array_equal(G.download().reshape(F.shape), F)
+
+
+def test_more_tiles_than_one_launch_holds():
+    """2^24 tiles of 256 threads exceed a launch: 258 tiles along z of 65535 one-cell-wide rows, 4.3 GB."""
+    ny, nz = 65535, 8225
+    F = np.arange(ny * nz, dtype=np.float64)
+    D, buf = chl.DeviceArray.from_host(F), chl.DeviceArray(F.size)
+    args = (1, ny, nz, 0, 1, ny, nz, -1)
+    chl.check(chl.lib().chl_pack_real_cells(D.ptr, buf.ptr, *args))
+    got = buf.download().reshape(ny, nz)
+    rows = np.r_[0:3, 3:ny - 3:509, ny - 3:ny]  # every launch's share, first and last rows whole
+    want = np.arange(nz, dtype=np.float64)[None, :] * ny + rows[:, None]
+    assert np.array_equal(got[rows], want)
+    del got
+    chl.check(chl.lib().chl_memcpy_dtod(D.ptr, buf.ptr, 8))  # spoil one element, then unpack over it
+    chl.check(chl.lib().chl_unpack_real_cells(buf.ptr, D.ptr, *args))
+    assert np.array_equal(D.download(), F)
